@@ -157,6 +157,9 @@ int fdtd_hip_grid_get_eps(fdtd_grid *g, int which, double *host);
 int fdtd_hip_grid_set_ns_coefs(fdtd_grid *g, const double *cells, double r_half);
 /* one reference update(): E/H halves, source, per-step NTFF */
 int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p);
+/* n update()s, p[i] the parameters of the i-th: the same results as n calls of
+ * fdtd_hip_grid_step; FP64 grids advance several steps per launch */
+int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n);
 /* which 0..8: TM Ez Jz Dz Hx Mx Bx Hy My By / TE Ex Jx Dx Ey Jy Dy Hz Mz Bz;
  * host buffers hold NPXa*NPYa complex doubles (re,im) in the solver layout */
 int fdtd_hip_grid_get_field(fdtd_grid *g, int which, double *host);

@@ -6,9 +6,11 @@
 //           (calcMB + calcH) -> per-step NTFF          (mpiTM_UPML.c:196-217, mpiTE_UPML.c:290-304)
 //   plain : H half -> E half (+ Gaussian pulse) -> ntff*_TimeCalc
 //                                                       (fdtdTM_upml.c:54-66, fdtdTE_upml.c:168-192)
-// The arithmetic of every update keeps the reference's operation order and is
-// compiled without FMA contraction, so results agree with the CPU solver to
-// rounding of the device sin/cos/exp only.
+// The arithmetic of every update here keeps the reference's operation order and
+// is compiled without FMA contraction, so results agree with the CPU solver to
+// rounding of the device sin/cos/exp only.  The UPML solvers' steps run in blocks
+// (fdtd_stream.hip), which agree to rounding; these kernels take over where a
+// grid's state, structure or wave is changed between steps.
 //
 // HBM layout: each complex field is an array of double2 (re, im), row-major
 // k = i*NPYa + j (j = y contiguous), exactly the reference's layout, so host
@@ -672,8 +674,8 @@ __global__ __launch_bounds__(256) void k_te_h(GridPtrs g, Tabs t)
 // ---------------------------------------------------------------- NTFF (time domain)
 
 // gather the contour samples of this step: E value (signed) and the averaged,
-// signed H value of every contour cell
-__global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Contour ct, double2 *cE, double2 *cH)
+// signed H value of every contour cell, sp elements per cell
+__global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Contour ct, int sp, double2 *cE, double2 *cH)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= ct.total) return;
@@ -689,8 +691,8 @@ __global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Co
   ev.y = sg.es * e.y;
   hv.x = sg.hs * (h0.x + h1.x);
   hv.y = sg.hs * (h0.y + h1.y);
-  cE[p] = ev;
-  cH[p] = hv;
+  cE[(size_t)p * sp] = ev;
+  cH[(size_t)p * sp] = hv;
 }
 
 #define NT_GUARD_DEV 4  // guard bins allocated before and after the accumulators
@@ -1353,6 +1355,7 @@ struct fdtd_grid {
   int NPXa, NPYa, off;
   size_t ncell;
   double2 *F[9];
+  double2 *F64;  // FP64 grids: the block that holds F[]
   double2 **Fdev;  // device copy of F[] for the gather kernel
   double *eps[3];
   double *tab;
@@ -1393,6 +1396,9 @@ struct fdtd_grid {
   double2 *tw;
   fdtd_model_state *mstate;
   FastState *fs;  // FP32 fused path (precision FDTD_FP32); F[] then serve as FP64 export buffers
+  StreamState *st;  // FP64 UPML grids: the blocked path
+  int general;      // the grid left it (since the last reset): every step runs the kernels that keep all auxiliaries
+  int auxok;        // the auxiliaries of the cells without UPML are in F
   double *nsc;    // NS flavour: [nns][ncell] per-cell coefficients (fdtd_hip_grid_set_ns_coefs)
   int nns;        // NS flavour: TM 5, TE 10 maps
   double ns_r2;   // NS flavour: r/2 of the second differences
@@ -1675,11 +1681,12 @@ static int dft_stage(fdtd_grid *g, int n, double time0, hipStream_t st)
   return col;
 }
 
-// contour samples of n inner steps of the FP32 kernel ([n][3][total] float2:
-// signed E, H on the side, H one cell back) -> the packing of k_ntff_gather,
+// contour samples of n inner steps of a fused kernel ([n][3][total], float2 or
+// double2: signed E, H on the side, H one cell back) -> the packing of k_ntff_gather,
 // step s of cell p at cE[s * ss + p * sp] (the binning's [cell][n], or the
 // DFT's staging [step][cell])
-__global__ __launch_bounds__(256) void k_ctr_combine(const float2 *smp, Contour ct, long ss, long sp, double2 *cE,
+template <class V>
+__global__ __launch_bounds__(256) void k_ctr_combine(const V *smp, Contour ct, long ss, long sp, double2 *cE,
                                                      double2 *cH)
 {
   const int p = blockIdx.x * 256 + threadIdx.x, s = blockIdx.y;
@@ -1687,8 +1694,8 @@ __global__ __launch_bounds__(256) void k_ctr_combine(const float2 *smp, Contour 
   int q = 0;
   while (q < 3 && p >= ct.s[q + 1].off) q++;
   const double hs = ct.s[q].hs;
-  const float2 *sm = smp + (size_t)s * 3 * ct.total;
-  const float2 e = sm[p], h0 = sm[ct.total + p], h1 = sm[2 * ct.total + p];
+  const V *sm = smp + (size_t)s * 3 * ct.total;
+  const V e = sm[p], h0 = sm[ct.total + p], h1 = sm[2 * ct.total + p];
   cE[(size_t)s * ss + (size_t)p * sp] = make_double2((double)e.x, (double)e.y);
   cH[(size_t)s * ss + (size_t)p * sp] = make_double2(hs * ((double)h0.x + (double)h1.x), hs * ((double)h0.y + (double)h1.y));
 }
@@ -1721,14 +1728,14 @@ static int grid_bin_samples(void *ctx, const float2 *samples, int n, const doubl
   const dim3 cgrid((g->ct.total + 255) / 256, n);
   if (g->ntn) {
     // binned step by step: [cell][nbuf], the first n steps of each cell; the DFT reads the same buffers
-    hipLaunchKernelGGL(k_ctr_combine, cgrid, dim3(256), 0, st, samples, g->ct, 1L, (long)g->nbuf, g->cE, g->cH);
+    hipLaunchKernelGGL(k_ctr_combine<float2>, cgrid, dim3(256), 0, st, samples, g->ct, 1L, (long)g->nbuf, g->cE, g->cH);
     HIPCHK(hipEventRecord(consumed, st));
     launch_bin(g, n, times[0], st);
     if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, n, (long)llround(times[0]) - 1, st);
   } else if (g->nf) {
     // DFT only: staged, the DFT runs over up to sCap steps at once
     const size_t col = (size_t)dft_stage(g, n, times[0], st) * g->ct.total;
-    hipLaunchKernelGGL(k_ctr_combine, cgrid, dim3(256), 0, st, samples, g->ct, (long)g->ct.total, 1L, g->sE + col,
+    hipLaunchKernelGGL(k_ctr_combine<float2>, cgrid, dim3(256), 0, st, samples, g->ct, (long)g->ct.total, 1L, g->sE + col,
                        g->sH + col);
     HIPCHK(hipEventRecord(consumed, st));
   } else {
@@ -1744,6 +1751,12 @@ static int ntff_sync(fdtd_grid *g)
 {
   if (g->ns) HIPCHK(hipStreamSynchronize(g->ns));
   return FDTD_OK;
+}
+
+// F[] from the block of an FP64 grid's state
+static void set_F64(fdtd_grid *g)
+{
+  for (int f = 0; f < 9; f++) g->F[f] = (double2 *)((char *)g->F64 + f * stream_stride(g->ncell));
 }
 
 extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
@@ -1775,9 +1788,11 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
   g->ncell = (size_t)g->NPXa * g->NPYa;
   *out = g;
   // the FP64 state; an FP32 grid uses these only as export buffers, made on first use
-  for (int f = 0; f < 9 && d->precision == FDTD_FP64; f++) {
-    HIPCHK(dev_malloc(&g->F[f], g->ncell * sizeof(double2)));
-    HIPCHK(hipMemset(g->F[f], 0, g->ncell * sizeof(double2)));
+  if (d->precision == FDTD_FP64) {
+    const size_t stride = stream_stride(g->ncell);
+    HIPCHK(dev_malloc(&g->F64, 9 * stride));
+    HIPCHK(hipMemset(g->F64, 0, 9 * stride));
+    set_F64(g);
   }
   HIPCHK(dev_malloc(&g->Fdev, 9 * sizeof(double2 *)));
   HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
@@ -1810,8 +1825,9 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
   std::vector<double> tab, mn, mx, ca, sa, cb, sb;
   build_time_shift(g, tab, mn, mx, ca, sa, cb, sb, d->ntff_time != 0);
   const int P = std::max(1, g->ct.total);
-  // FP32 grids bin a whole block of steps at once: sample buffers for FAST_MAX_T steps
-  g->nbuf = d->precision == FDTD_FP32 ? FAST_MAX_T : 1;
+  // blocked paths bin a whole block of steps at once: sample buffers for as many
+  const bool upml = d->flavour == FDTD_FLAVOUR_MPI || d->flavour == FDTD_FLAVOUR_PLAIN;
+  g->nbuf = d->precision == FDTD_FP32 ? FAST_MAX_T : (upml ? STREAM_T : 1);
   // the sample buffer: E samples of every cell, then H, nbuf steps per cell
   // (the binning's records address both from cE)
   HIPCHK(dev_malloc(&g->cE, (size_t)2 * g->nbuf * P * sizeof(double2)));
@@ -1835,6 +1851,16 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
   HIPCHK(dev_malloc(&g->spec, 321 * 360 * sizeof(double)));
   HIPCHK(dev_malloc(&g->tw, 4096 * sizeof(double2)));
   HIPCHK(dev_malloc(&g->mstate, sizeof(fdtd_model_state)));
+  g->auxok = 1;
+  if (d->precision == FDTD_FP64 && upml) {
+    int rc = stream_create(*d, g->off, g->ct, &g->st);
+    if (rc == FDTD_ENOMEM) {
+      stream_destroy(g->st);
+      g->st = nullptr;
+    } else if (rc) {
+      return rc;
+    }
+  }
   if (d->precision == FDTD_FP32) {
     int rc = fast_state_create(*d, &g->fs);
     if (rc) return rc;
@@ -1903,7 +1929,8 @@ extern "C" int fdtd_hip_grid_destroy(fdtd_grid *g)
     (void)hipEventDestroy(g->ev_k);
     g->ns = nullptr;
   }
-  for (int f = 0; f < 9; f++) (void)dev_free(g->F[f]);
+  for (int f = 0; f < 9 && !g->F64; f++) (void)dev_free(g->F[f]);
+  (void)dev_free(g->F64);
   (void)dev_free(g->Fdev);
   for (int e = 0; e < 3; e++) (void)dev_free(g->eps[e]);
   (void)dev_free(g->nsc);
@@ -1930,13 +1957,37 @@ extern "C" int fdtd_hip_grid_destroy(fdtd_grid *g)
   (void)dev_free(g->tw);
   (void)dev_free(g->mstate);
   fast_state_destroy(g->fs);
+  stream_destroy(g->st);
   delete g;
+  return FDTD_OK;
+}
+
+// the auxiliaries the blocked FP64 path does not keep, formed in F
+static int ensure_aux(fdtd_grid *g)
+{
+  if (!g->st || g->auxok) return FDTD_OK;
+  int rc = stream_fill_aux(g->st, g->F64);
+  if (rc == FDTD_OK) g->auxok = 1;
+  return rc;
+}
+
+// from here on (to the next reset) step by step, keeping every auxiliary; `steps_only`:
+// only if steps were taken
+static int go_general(fdtd_grid *g, bool steps_only)
+{
+  if (!g->st || g->general || (steps_only && !stream_steps_done(g->st))) return FDTD_OK;
+  int rc = ensure_aux(g);
+  if (rc) return rc;
+  g->general = 1;
+  HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
   return FDTD_OK;
 }
 
 extern "C" int fdtd_hip_grid_set_coefs(fdtd_grid *g, const fdtd_coef_tables *t)
 {
   if (!g || !t) return fdtd_fail(FDTD_EINVAL, "null argument");
+  int rc0 = go_general(g, true);
+  if (rc0) return rc0;
   const size_t nx = g->d.N_PX, ny = g->d.N_PY;
   for (int q = 0; q < 5; q++) {
     if (!t->x[q]) return fdtd_fail(FDTD_EINVAL, "missing x table %d", q);
@@ -1950,6 +2001,7 @@ extern "C" int fdtd_hip_grid_set_coefs(fdtd_grid *g, const fdtd_coef_tables *t)
   HIPCHK(hipMemcpy((void *)g->tabs.sx, t->sx, nx * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy((void *)g->tabs.sy, t->sy, ny * sizeof(double), hipMemcpyHostToDevice));
   if (g->fs) return fast_state_set_coefs(g->fs, t);
+  if (g->st) return stream_set_coefs(g->st, t);
   return FDTD_OK;
 }
 
@@ -1965,6 +2017,8 @@ extern "C" int fdtd_hip_grid_set_ns_coefs(fdtd_grid *g, const double *cells, dou
 extern "C" int fdtd_hip_grid_fill_eps(fdtd_grid *g, const fdtd_model_state *m)
 {
   if (!g || !m) return fdtd_fail(FDTD_EINVAL, "null argument");
+  int rc0 = go_general(g, true);
+  if (rc0) return rc0;
   HIPCHK(hipMemcpy(g->mstate, m, sizeof(*m), hipMemcpyHostToDevice));
   dim3 blk(64, 4), grd((g->NPYa + 63) / 64, (g->NPXa + 3) / 4);
   hipLaunchKernelGGL(k_fill_eps, grd, blk, 0, 0, g->mstate, g->eps[0], g->eps[1], g->eps[2], g->NPXa, g->NPYa, g->off,
@@ -1974,14 +2028,18 @@ extern "C" int fdtd_hip_grid_fill_eps(fdtd_grid *g, const fdtd_model_state *m)
   HIPCHK(hipGetLastError());
   HIPCHK(hipDeviceSynchronize());
   if (g->fs) return fast_state_set_inv_eps(g->fs, g->eps, g->NPYa, g->off);
+  if (g->st) return stream_set_eps(g->st, g->eps);
   return FDTD_OK;
 }
 
 extern "C" int fdtd_hip_grid_set_eps(fdtd_grid *g, int which, const double *host)
 {
   if (!g || !host || which < 0 || which > 2) return fdtd_fail(FDTD_EINVAL, "bad argument");
+  int rc0 = go_general(g, true);
+  if (rc0) return rc0;
   HIPCHK(hipMemcpy(g->eps[which], host, g->ncell * sizeof(double), hipMemcpyHostToDevice));
   if (g->fs) return fast_state_set_inv_eps(g->fs, g->eps, g->NPYa, g->off);
+  if (g->st) return stream_set_eps(g->st, g->eps);
   return FDTD_OK;
 }
 
@@ -1992,6 +2050,55 @@ extern "C" int fdtd_hip_grid_get_eps(fdtd_grid *g, int which, double *host)
   return FDTD_OK;
 }
 
+// n (<= STREAM_T) consecutive steps of an FP64 UPML grid in one launch, and the NTFF
+// work of all of them
+static int stream_block(fdtd_grid *g, const fdtd_step_params *p, int n)
+{
+  const bool ctr = g->ct.total > 0 && (g->ntn || g->nf);
+  const double2 *smp = nullptr;
+  int rc = stream_steps(g->st, &g->F64, p, n, ctr ? 1 : 0, &smp);
+  if (rc) return rc;
+  set_F64(g);
+  g->auxok = 0;
+  if (!ctr) return FDTD_OK;
+  const dim3 cgrid((g->ct.total + 255) / 256, n);
+  if (g->ntn) {
+    hipLaunchKernelGGL(k_ctr_combine<double2>, cgrid, dim3(256), 0, 0, smp, g->ct, 1L, (long)g->nbuf, g->cE, g->cH);
+    launch_bin(g, n, p[0].time, 0);
+    if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, n, (long)llround(p[0].time) - 1, 0);
+  } else {
+    const size_t col = (size_t)dft_stage(g, n, p[0].time, 0) * g->ct.total;
+    hipLaunchKernelGGL(k_ctr_combine<double2>, cgrid, dim3(256), 0, 0, smp, g->ct, (long)g->ct.total, 1L, g->sE + col,
+                       g->sH + col);
+  }
+  HIPCHK(hipGetLastError());
+  return FDTD_OK;
+}
+
+extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n)
+{
+  if (!g || !p || n < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
+  for (int i = 0; i < n;) {
+    int rc, m = 1;
+    if (g->st && !g->general && stream_follows(g->st, p + i)) {
+      const fdtd_step_params &a = p[i];
+      while (m < STREAM_T && i + m < n) {
+        const fdtd_step_params &b = p[i + m];
+        if (b.time != a.time + m || b.angle_deg != a.angle_deg || b.k != a.k || b.omega != a.omega || b.dot_x != a.dot_x ||
+            b.dot_y != a.dot_y || b.use_x != a.use_x || b.use_y != a.use_y)
+          break;
+        m++;
+      }
+      rc = stream_block(g, p + i, m);
+    } else {
+      rc = fdtd_hip_grid_step(g, p + i);
+    }
+    if (rc) return rc;
+    i += m;
+  }
+  return FDTD_OK;
+}
+
 extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
 {
   if (!g || !p) return fdtd_fail(FDTD_EINVAL, "null argument");
@@ -1999,6 +2106,11 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
   if (g->fs) {
     int launched = 0;
     return fast_state_step(g->fs, p, &launched);
+  }
+  if (g->st && !g->general) {
+    if (stream_follows(g->st, p)) return stream_block(g, p, 1);
+    int rc = go_general(g, false);
+    if (rc) return rc;
   }
   GridPtrs gp;
   for (int f = 0; f < 9; f++) gp.F[f] = g->F[f];
@@ -2091,14 +2203,14 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
   HIPCHK(hipGetLastError());
   if (g->ntn && g->ct.total > 0) {
     hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, (const double2 *const *)g->Fdev,
-                       g->ct, g->cE, g->cH);
+                       g->ct, g->nbuf, g->cE, g->cH);
     launch_bin(g, 1, p->time, 0);
-    if (g->nf) dft_add(g, g->cE, g->cH, 1, 1, 1, (long)llround(p->time) - 1, 0);
+    if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, 1, (long)llround(p->time) - 1, 0);
     HIPCHK(hipGetLastError());
   } else if (g->nf && g->ct.total > 0) {
     const size_t col = (size_t)dft_stage(g, 1, p->time, 0) * g->ct.total;
     hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, (const double2 *const *)g->Fdev,
-                       g->ct, g->sE + col, g->sH + col);
+                       g->ct, 1, g->sE + col, g->sH + col);
     HIPCHK(hipGetLastError());
   }
   return FDTD_OK;
@@ -2123,6 +2235,7 @@ extern "C" int fdtd_hip_grid_get_field(fdtd_grid *g, int which, double *host)
     int rc = fast_state_export(g->fs, which, g->F[which], g->NPYa, g->off);
     if (rc) return rc;
   }
+  if (which % 3 && (rc0 = ensure_aux(g))) return rc0;
   HIPCHK(hipMemcpy(host, g->F[which], g->ncell * sizeof(double2), hipMemcpyDeviceToHost));
   return FDTD_OK;
 }
@@ -2131,7 +2244,7 @@ extern "C" int fdtd_hip_grid_set_field(fdtd_grid *g, int which, const double *ho
 {
   if (!g || !host || which < 0 || which > 8) return fdtd_fail(FDTD_EINVAL, "bad argument");
   int rc0 = ensure_F(g, which);
-  if (rc0) return rc0;
+  if (rc0 || (rc0 = go_general(g, false))) return rc0;
   HIPCHK(hipMemcpy(g->F[which], host, g->ncell * sizeof(double2), hipMemcpyHostToDevice));
   if (g->fs) return fast_state_import(g->fs, which, g->F[which], g->NPYa, g->off);
   return FDTD_OK;
@@ -2162,6 +2275,9 @@ extern "C" int fdtd_hip_grid_reset(fdtd_grid *g)
   }
   g->sFill = 0;
   HIPCHK(hipDeviceSynchronize());
+  if (g->st) stream_reset(g->st);
+  g->general = 0;
+  g->auxok = 1;
   if (g->fs) return fast_state_reset(g->fs);
   return FDTD_OK;
 }

@@ -55,6 +55,7 @@ struct FastStep {
   float pad;
 };
 
+#define STREAM_T 8  // steps per launch of the FP64 UPML path
 #define FAST_MAX_T 16
 // rows of a UPML tile's block: the 4-wavefront UPML body (4 x 8 rows, the
 // merged, split and two-stream shapes, and batches) and the wide bodies of the
@@ -135,6 +136,24 @@ struct FastArgs {
   FastContour ct;
   FastStep st[FAST_MAX_T];  // single-instance runs: the block's steps, passed by value
 };
+
+// ---------------------------------------------------------------- FP64 blocked path
+// (fdtd_stream.hip) of the UPML solvers; the grid owns the current arrays F, the
+// state the other buffers.  stream_follows: whether a step continues the steps
+// taken so far; a grid whose fields, structure or wave were changed in between
+// goes on step by step with the kernels that keep every auxiliary.
+struct StreamState;
+// bytes between the nine arrays of an FP64 state of n cells, which lie in one block
+static inline size_t stream_stride(size_t n) { return (n * sizeof(double2) + 255) & ~(size_t)255; }
+int stream_create(const fdtd_grid_desc &d, int off, const Contour &ct, StreamState **out);
+void stream_destroy(StreamState *s);
+int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t);
+int stream_set_eps(StreamState *s, double *const *eps);
+void stream_reset(StreamState *s);
+long stream_steps_done(const StreamState *s);
+bool stream_follows(const StreamState *s, const fdtd_step_params *p);
+int stream_steps(StreamState *s, double2 **F, const fdtd_step_params *p, int n, int samples, const double2 **smp);
+int stream_fill_aux(StreamState *s, double2 *F);
 
 struct FastState;
 int fast_state_create(const fdtd_grid_desc &d, FastState **out);

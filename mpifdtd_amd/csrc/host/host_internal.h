@@ -18,5 +18,8 @@ FDTD_HIDDEN int fdtd_hip_grid_far_field_noalloc(fdtd_grid *g, double k, double c
                                                 double *out360);
 /* far-field coefficient sqrt(i k / (8 pi R0)) e^{i k R0} of the current field globals */
 FDTD_HIDDEN double complex solver_ff_coef(void);
+/* up to n steps of the solver that `update` belongs to, handed to the device
+   together; the number taken, 0 where the caller has to step one by one */
+FDTD_HIDDEN int solver_run(void (*update)(void), int n);
 
 #endif

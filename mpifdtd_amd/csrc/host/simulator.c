@@ -16,6 +16,7 @@
 #include "mpifdtd_models.h"
 #include "mpifdtd_simulator.h"
 #include "mpifdtd_solvers.h"
+#include "host_internal.h"
 
 static fdtd_method update_ = NULL, init_ = NULL, finish_ = NULL, reset_ = NULL;
 static fdtd_dcomplex *(*draw_)(void) = NULL;
@@ -152,8 +153,13 @@ double *simulator_getEps(void) { return (*eps_)(); }
 /* n x simulator_calc() without returning to the caller in between */
 void fdtd_simulator_run(int nsteps)
 {
-  for (int n = 0; n < nsteps; n++) {
-    (*update_)();
-    field_nextStep();
+  while (nsteps > 0) {
+    int n = solver_run(update_, nsteps);
+    if (n == 0) {
+      (*update_)();
+      field_nextStep();
+      n = 1;
+    }
+    nsteps -= n;
   }
 }

@@ -55,6 +55,8 @@ static int finite_every_ = 0, finite_abort_ = 0, finite_since_ = 0;
 static int finite_step_ = -1;
 static long long finite_count_ = 0;
 
+#define RUN_STEPS 64 /* steps handed to the device per call of solver_run */
+
 static const int slot_of_[3] = {0, 3, 6};
 
 static void die(const char *what)
@@ -414,10 +416,9 @@ static void solver_init(int kind)
   finite_count_ = 0;
 }
 
-static void solver_update(int kind)
+/* the parameters of the step at the current field time */
+static fdtd_step_params step_params(int kind)
 {
-  solver_t *s = &slv_[kind];
-  if (!s->g) { fprintf(stderr, "mpifdtd_amd: update before init\n"); exit(2); }
   fdtd_step_params p;
   memset(&p, 0, sizeof p);
   p.time = field_getTime();
@@ -439,6 +440,14 @@ static void solver_update(int kind)
     p.use_x = co != 0.0;
     p.use_y = si != 0.0;
   }
+  return p;
+}
+
+static void solver_update(int kind)
+{
+  solver_t *s = &slv_[kind];
+  if (!s->g) { fprintf(stderr, "mpifdtd_amd: update before init\n"); exit(2); }
+  const fdtd_step_params p = step_params(kind);
   CHECK(fdtd_hip_grid_step(s->g, &p));
   if (finite_every_ > 0 && ++finite_since_ >= finite_every_) {
     finite_since_ = 0;
@@ -701,6 +710,25 @@ int fdtd_solver_dims(int out[4])
   return FDTD_OK;
 }
 
+static int kind_of(fdtd_method update);
+
+/* up to n steps of the solver that `update` belongs to, field_nextStep after each,
+   handed to the device together; returns how many were taken, 0 where the caller
+   has to step (a finite check runs between steps) */
+int solver_run(fdtd_method update, int n)
+{
+  const int kind = kind_of(update);
+  if (kind < 0 || !slv_[kind].g || slv_[kind].blocked || finite_every_ > 0) return 0;
+  fdtd_step_params p[RUN_STEPS];
+  if (n > RUN_STEPS) n = RUN_STEPS;
+  for (int i = 0; i < n; i++) {
+    p[i] = step_params(kind);
+    field_nextStep();
+  }
+  CHECK(fdtd_hip_grid_steps(slv_[kind].g, p, n));
+  return n;
+}
+
 /* ---------------------------------------------------------------- MPI TM */
 static void mpi_tm_init(void) { solver_init(SLV_MPI_TM); }
 static void mpi_tm_update(void) { solver_update(SLV_MPI_TM); }
@@ -873,3 +901,16 @@ fdtd_dcomplex *fdtdTE_upml_getEx(void) { return (fdtd_dcomplex *)solver_field(SL
 fdtd_dcomplex *fdtdTE_upml_getEy(void) { return (fdtd_dcomplex *)solver_field(SLV_TE, 1); }
 fdtd_dcomplex *fdtdTE_upml_getHz(void) { return (fdtd_dcomplex *)solver_field(SLV_TE, 2); }
 double *fdtdTE_upml_getEps(void) { return solver_eps(SLV_TE); }
+
+static int kind_of(fdtd_method update)
+{
+  if (update == mpi_tm_update) return SLV_MPI_TM;
+  if (update == mpi_te_update) return SLV_MPI_TE;
+  if (update == tm_update) return SLV_TM;
+  if (update == te_update) return SLV_TE;
+  if (update == split_tm_update) return SLV_SPLIT_TM;
+  if (update == split_te_update) return SLV_SPLIT_TE;
+  if (update == ns_tm_update) return SLV_NS_TM;
+  if (update == ns_te_update) return SLV_NS_TE;
+  return -1;
+}
