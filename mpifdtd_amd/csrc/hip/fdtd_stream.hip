@@ -20,7 +20,7 @@
 // cells without UPML the auxiliaries are formed from the fields as a row is
 // loaded.  What bounds it: the chain of a row's dependent FP64 operations, LDS
 // hand-ons and one barrier per row (the two kernels keep their SIMDs about 45 %
-// active, waves waiting 40-50 % of the time), at 2.7 us a step on 1056 x 1056 where the
+// active, waves waiting 40-50 % of the time), at 7.3 us a step on 1056 x 1056 where the
 // two-launch step that reads and writes every array took 57 (8-step launches of
 // 58.5 us, TM; two columns a lane: one took 38.0 + 45.4 us in two launches).
 // Physics per step as in the reference (mpiTM_UPML.c:196-217,
