@@ -155,6 +155,9 @@ int fdtd_hip_grid_get_eps(fdtd_grid *g, int which, double *host);
  * r_half is r/2 of the second differences, r = 1/6 + k^2/180 - k^4/23040
  * (nsFdtdTM.c:117-118, nsFdtdTE.c:255-256) */
 int fdtd_hip_grid_set_ns_coefs(fdtd_grid *g, const double *cells, double r_half);
+/* the same maps formed on the device from the grid's eps maps: sig = sig_max sigma
+ * at i, i + 1/2 (N_PX values each), j and j + 1/2 (N_PY) */
+int fdtd_hip_grid_form_ns_coefs(fdtd_grid *g, const double *const sig[4], double omega, double k, double r_half);
 /* one reference update(): E/H halves, source, per-step NTFF */
 int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p);
 /* n update()s, p[i] the parameters of the i-th: the same results as n calls of

@@ -1397,7 +1397,9 @@ struct fdtd_grid {
   fdtd_model_state *mstate;
   FastState *fs;  // FP32 fused path (precision FDTD_FP32); F[] then serve as FP64 export buffers
   StreamState *st;  // FP64 UPML grids: the blocked path
+  SplitState *sp;   // FP64 split-field and NS grids: theirs
   int general;      // the grid left it (since the last reset): every step runs the kernels that keep all auxiliaries
+  int epsok;        // the eps maps are set
   int auxok;        // the auxiliaries of the cells without UPML are in F
   double *nsc;    // NS flavour: [nns][ncell] per-cell coefficients (fdtd_hip_grid_set_ns_coefs)
   int nns;        // NS flavour: TM 5, TE 10 maps
@@ -1861,6 +1863,15 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
       return rc;
     }
   }
+  if (d->precision == FDTD_FP64 && !upml) {
+    int rc = split_create(*d, &g->sp);
+    if (rc == FDTD_ENOMEM) {
+      split_destroy(g->sp);
+      g->sp = nullptr;
+    } else if (rc) {
+      return rc;
+    }
+  }
   if (d->precision == FDTD_FP32) {
     int rc = fast_state_create(*d, &g->fs);
     if (rc) return rc;
@@ -1958,6 +1969,7 @@ extern "C" int fdtd_hip_grid_destroy(fdtd_grid *g)
   (void)dev_free(g->mstate);
   fast_state_destroy(g->fs);
   stream_destroy(g->st);
+  split_destroy(g->sp);
   delete g;
   return FDTD_OK;
 }
@@ -1975,6 +1987,11 @@ static int ensure_aux(fdtd_grid *g)
 // only if steps were taken
 static int go_general(fdtd_grid *g, bool steps_only)
 {
+  // the split solvers' blocks form the sums from the split components, which a caller may set apart
+  if (g->sp && !steps_only && !g->general) {
+    g->general = 1;
+    HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
+  }
   if (!g->st || g->general || (steps_only && !stream_steps_done(g->st))) return FDTD_OK;
   int rc = ensure_aux(g);
   if (rc) return rc;
@@ -2002,6 +2019,11 @@ extern "C" int fdtd_hip_grid_set_coefs(fdtd_grid *g, const fdtd_coef_tables *t)
   HIPCHK(hipMemcpy((void *)g->tabs.sy, t->sy, ny * sizeof(double), hipMemcpyHostToDevice));
   if (g->fs) return fast_state_set_coefs(g->fs, t);
   if (g->st) return stream_set_coefs(g->st, t);
+  if (g->sp) {
+    int rc = split_set_coefs(g->sp, t);
+    if (rc) return rc;
+    return g->epsok ? split_set_eps(g->sp, g->eps, g->tabs.x[0], g->tabs.y[0]) : FDTD_OK;
+  }
   return FDTD_OK;
 }
 
@@ -2011,6 +2033,81 @@ extern "C" int fdtd_hip_grid_set_ns_coefs(fdtd_grid *g, const double *cells, dou
   if (g->d.flavour != FDTD_FLAVOUR_NS) return fdtd_fail(FDTD_EINVAL, "per-cell NS coefficients need the NS flavour");
   HIPCHK(hipMemcpy(g->nsc, cells, g->nns * g->ncell * sizeof(double), hipMemcpyHostToDevice));
   g->ns_r2 = r_half;
+  if (g->sp) return split_set_ns(g->sp, g->nsc, r_half);
+  return FDTD_OK;
+}
+
+// nsFdtdTM.c:226-306 / nsFdtdTE.c:100-181 and field.c:155-177: the per-cell
+// coefficients of the NS solvers from the eps maps, each with the reference's
+// expression.  x0, x1 (y0, y1): sig_max sigma at i and i + 1/2 (j and j + 1/2).
+// On one host core these cost 80 ms for the ten TE maps of 1056 x 1056 cells, more
+// than a thousand of its steps; here they are formed where they are used.
+__device__ __forceinline__ double ns_beta(double alpha)
+{
+  const double t = tanh(alpha);
+  return t / (1 + t * t);
+}
+__device__ __forceinline__ double ns_coef1(double b) { return (1 - b) / (1 + b); }
+__device__ __forceinline__ double ns_wave_factor(double eps, double w_s, double k_s)
+{
+  const double nn = sqrt(eps);
+  const double u0 = sin(w_s * 0.5) / sin(k_s * 0.5), u1 = sin(w_s * 0.5) / sin(nn * k_s * 0.5);
+  const double _n = u0 / u1;
+  return 1.0 / (_n * nn) - 1.0;  // exactly 0 where n = 1
+}
+__global__ __launch_bounds__(256) void k_ns_form(const double *e0, const double *e1, const double *e2, const double *x0,
+                                                 const double *x1, const double *y0, const double *y1, int tm, int nx, int ny,
+                                                 double mu0, double w_s, double k_s, double *c)
+{
+  const int j = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
+  if (i >= nx || j >= ny) return;
+  const size_t n = (size_t)nx * ny, k = (size_t)i * ny + j;
+  // u z and u / z of a cell of permittivity e
+  const double sw = sin(w_s * 0.5);
+  auto u = [&](double e) { return sw / sin(k_s * sqrt(e) * 0.5); };
+  if (tm) {
+    const double b_ez_x = ns_beta(x0[i] / 2), b_hy_x = ns_beta(x1[i] / 2), b_hx_y = ns_beta(y1[j] / 2);
+    const double ez = u(e0[k]) * sqrt(mu0 / e0[k]) / (1 + b_ez_x);
+    c[k] = ez;      // C_EZXLX
+    c[n + k] = ez;  // C_EZYLY: b_ez_x, as nsFdtdTM.c:282 has it
+    c[2 * n + k] = u(e1[k]) / sqrt(mu0 / e1[k]) / (1.0 + b_hx_y);  // C_HXLY
+    c[3 * n + k] = u(e2[k]) / sqrt(mu0 / e2[k]) / (1.0 + b_hy_x);  // C_HYLX
+    c[4 * n + k] = ns_wave_factor(e0[k], w_s, k_s);
+    return;
+  }
+  if (i < 1 || j < 1 || i >= nx - 1 || j >= ny - 1) return;  // the reference leaves the border unset
+  const double e_ex = e0[k], e_ey = e1[k], e_hz = e2[k];
+  const double b_ex_y = ns_beta(y0[j] / (2 * e_ex)), b_ey_x = ns_beta(x0[i] / (2 * e_ey));
+  const double b_hz_x = ns_beta(x1[i] / (2 * e_hz)), b_hz_y = ns_beta(y1[j] / (2 * e_hz));
+  const double hz = u(e_hz) / sqrt(mu0 / e_hz);
+  c[k] = ns_coef1(b_ex_y);                                          // C_EX
+  c[n + k] = u(e_ex) * sqrt(mu0 / e_ex) / (1.0 + b_ex_y);           // C_EXLY
+  c[2 * n + k] = ns_coef1(b_ey_x);                                  // C_EY
+  c[3 * n + k] = u(e_ey) * sqrt(mu0 / e_ey) / (1.0 + b_ey_x);       // C_EYLX
+  c[4 * n + k] = ns_coef1(b_hz_x);                                  // C_HZX
+  c[5 * n + k] = hz / (1.0 + b_hz_x);                               // C_HZXLX
+  c[6 * n + k] = ns_coef1(b_hz_y);                                  // C_HZY
+  c[7 * n + k] = hz / (1.0 + b_hz_y);                               // C_HZYLY
+  c[8 * n + k] = ns_wave_factor(e_ex, w_s, k_s);
+  c[9 * n + k] = ns_wave_factor(e_ey, w_s, k_s);
+}
+
+extern "C" int fdtd_hip_grid_form_ns_coefs(fdtd_grid *g, const double *const sig[4], double omega, double k, double r_half)
+{
+  if (!g || !sig || !sig[0] || !sig[1] || !sig[2] || !sig[3]) return fdtd_fail(FDTD_EINVAL, "null argument");
+  if (g->d.flavour != FDTD_FLAVOUR_NS) return fdtd_fail(FDTD_EINVAL, "per-cell NS coefficients need the NS flavour");
+  const int nx = g->d.N_PX, ny = g->d.N_PY;
+  double *t = nullptr;
+  HIPCHK(dev_malloc(&t, 2 * (size_t)(nx + ny) * sizeof(double)));
+  double *const at[4] = {t, t + nx, t + 2 * nx, t + 2 * nx + ny};
+  for (int q = 0; q < 4; q++)
+    HIPCHK(hipMemcpy(at[q], sig[q], (size_t)(q < 2 ? nx : ny) * sizeof(double), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_ns_form, dim3((ny + 63) / 64, (nx + 3) / 4), dim3(64, 4), 0, 0, g->eps[0], g->eps[1], g->eps[2], at[0],
+                     at[1], at[2], at[3], g->d.mode == FDTD_MODE_TM ? 1 : 0, nx, ny, g->d.mu0, omega, k, g->nsc);
+  HIPCHK(hipGetLastError());
+  HIPCHK(dev_free(t));
+  g->ns_r2 = r_half;
+  if (g->sp) return split_set_ns(g->sp, g->nsc, r_half);
   return FDTD_OK;
 }
 
@@ -2029,6 +2126,8 @@ extern "C" int fdtd_hip_grid_fill_eps(fdtd_grid *g, const fdtd_model_state *m)
   HIPCHK(hipDeviceSynchronize());
   if (g->fs) return fast_state_set_inv_eps(g->fs, g->eps, g->NPYa, g->off);
   if (g->st) return stream_set_eps(g->st, g->eps);
+  g->epsok = 1;
+  if (g->sp) return split_set_eps(g->sp, g->eps, g->tabs.x[0], g->tabs.y[0]);
   return FDTD_OK;
 }
 
@@ -2040,6 +2139,8 @@ extern "C" int fdtd_hip_grid_set_eps(fdtd_grid *g, int which, const double *host
   HIPCHK(hipMemcpy(g->eps[which], host, g->ncell * sizeof(double), hipMemcpyHostToDevice));
   if (g->fs) return fast_state_set_inv_eps(g->fs, g->eps, g->NPYa, g->off);
   if (g->st) return stream_set_eps(g->st, g->eps);
+  g->epsok = 1;
+  if (g->sp) return split_set_eps(g->sp, g->eps, g->tabs.x[0], g->tabs.y[0]);
   return FDTD_OK;
 }
 
@@ -2075,12 +2176,24 @@ static int stream_block(fdtd_grid *g, const fdtd_step_params *p, int n)
   return FDTD_OK;
 }
 
+// n (<= split_depth) steps of a split-field or NS grid in one launch
+static int split_block(fdtd_grid *g, const fdtd_step_params *p, int n)
+{
+  int rc = split_steps(g->sp, &g->F64, p, n);
+  if (rc == FDTD_OK) set_F64(g);
+  return rc;
+}
+
 extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n)
 {
   if (!g || !p || n < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
+  const int depth = g->sp && !g->general ? split_depth(g->sp) : 0;
   for (int i = 0; i < n;) {
     int rc, m = 1;
-    if (g->st && !g->general && stream_follows(g->st, p + i)) {
+    if (depth && !g->nf) {
+      while (m < depth && i + m < n && p[i + m].angle_deg == p[i].angle_deg && p[i + m].k == p[i].k) m++;
+      rc = split_block(g, p + i, m);
+    } else if (g->st && !g->general && stream_follows(g->st, p + i)) {
       const fdtd_step_params &a = p[i];
       while (m < STREAM_T && i + m < n) {
         const fdtd_step_params &b = p[i + m];
@@ -2107,6 +2220,7 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
     int launched = 0;
     return fast_state_step(g->fs, p, &launched);
   }
+  if (g->sp && !g->general && !g->nf && split_depth(g->sp)) return split_block(g, p, 1);
   if (g->st && !g->general) {
     if (stream_follows(g->st, p)) return stream_block(g, p, 1);
     int rc = go_general(g, false);
@@ -2447,6 +2561,8 @@ extern "C" int fdtd_hip_grid_set_dft(fdtd_grid *g, const double *omega, int nf)
   if (!g || (nf > 0 && !omega) || nf < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
   if (nf > 0 && g->ct.total <= 0) return fdtd_fail(FDTD_ESTATE, "the grid has no NTFF contour");
   int rc;
+  // the split solvers' blocks take no contour samples
+  if (nf > 0 && g->sp && (rc = go_general(g, false))) return rc;
   if (g->fs && (rc = fast_state_flush(g->fs))) return rc;
   HIPCHK(hipDeviceSynchronize());
   (void)dev_free(g->dftOmega);

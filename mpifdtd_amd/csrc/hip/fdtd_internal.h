@@ -155,6 +155,18 @@ bool stream_follows(const StreamState *s, const fdtd_step_params *p);
 int stream_steps(StreamState *s, double2 **F, const fdtd_step_params *p, int n, int samples, const double2 **smp);
 int stream_fill_aux(StreamState *s, double2 *F);
 
+// the same for the split-field and non-standard solvers (fdtd_stream_split.hip), whose
+// state carries nothing of the step before: any steps may follow each other.
+// split_depth: steps per launch, 0 until the coefficients are set
+struct SplitState;
+int split_create(const fdtd_grid_desc &d, SplitState **out);
+void split_destroy(SplitState *s);
+int split_set_coefs(SplitState *s, const fdtd_coef_tables *t);
+int split_set_eps(SplitState *s, double *const *eps, const double *sx, const double *sy);
+int split_set_ns(SplitState *s, const double *nsc, double r2);
+int split_depth(const SplitState *s);
+int split_steps(SplitState *s, double2 **F, const fdtd_step_params *p, int n);
+
 struct FastState;
 int fast_state_create(const fdtd_grid_desc &d, FastState **out);
 void fast_state_destroy(FastState *s);

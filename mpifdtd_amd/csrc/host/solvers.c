@@ -140,98 +140,28 @@ int fdtd_solver_finiteStatus(int *step, long long *count)
 static double ns_beta(double alpha) { return tanh(alpha) / (1 + pow(tanh(alpha), 2)); }
 static double ns_coef1(double beta) { return (1 - beta) / (1 + beta); }
 
-/* the factor 1/(_n n) - 1 of field_nsScatteredWaveNotUPML (field.c:155-177),
-   exactly 0 where n = 1 */
-static double ns_wave_factor(double eps, double eps0, double w_s, double k_s)
-{
-  const double nn = sqrt(eps / eps0);
-  const double u0 = sin(w_s * 0.5) / sin(k_s * 0.5), u1 = sin(w_s * 0.5) / sin(nn * k_s * 0.5);
-  const double _n = u0 / u1;
-  return 1.0 / (_n * nn) - 1.0;
-}
-
-/* nsFdtdTE.c:100-181: all ten TE maps from EPS_EX, EPS_HZ and EPS_EY, over the
-   interior cells the reference fills (the border stays zero) */
-static void ns_te_cells(const double *eps, double *cell, size_t n)
+/* the per-cell coefficients of the NS solvers (nsFdtdTM.c:226-306, nsFdtdTE.c:100-181),
+   formed on the device from the eps maps and these conductivities */
+static int build_ns_coefs(fdtd_grid *g)
 {
   const int nx = N_PX, ny = N_PY;
-  const double R = 1.0e-8, M = 2.0, eps0 = 1.0, C = field_getLightSpeed(), mu0 = field_getMu0();
+  double *t = (double *)malloc(2 * ((size_t)nx + ny) * sizeof(double));
+  if (!t) return FDTD_ENOMEM;
+  const double R = 1.0e-8, M = 2.0, eps0 = 1.0, C = field_getLightSpeed();
   const double sig_max = -(M + 1.0) * eps0 * C / N_PML * log(R);
-  const double w_s = field_getOmega(), k_s = field_getK();
-  memset(cell, 0, 10 * n * sizeof(double));
-  for (int i = 1; i < nx - 1; i++) {
-    for (int j = 1; j < ny - 1; j++) {
-      const size_t k = (size_t)i * ny + j;
-      const double e_ex = eps[k], e_ey = eps[n + k], e_hz = eps[2 * n + k];
-      const double sig_ex_y = sig_max * field_sigmaY(i + 0.5, j), sig_ey_x = sig_max * field_sigmaX(i, j + 0.5);
-      const double sig_hz_x = sig_max * field_sigmaX(i + 0.5, j + 0.5), sig_hz_y = sig_max * field_sigmaY(i + 0.5, j + 0.5);
-      const double b_ex_y = ns_beta(sig_ex_y / (2 * e_ex)), b_ey_x = ns_beta(sig_ey_x / (2 * e_ey));
-      const double b_hz_x = ns_beta(sig_hz_x / (2 * e_hz)), b_hz_y = ns_beta(sig_hz_y / (2 * e_hz));
-      const double z_hz = sqrt(mu0 / e_hz), n_hz = sqrt(e_hz / eps0);
-      const double u_hz = sin(w_s * 0.5) / sin(k_s * n_hz * 0.5);
-      cell[4 * n + k] = ns_coef1(b_hz_x);                  /* C_HZX */
-      cell[5 * n + k] = u_hz / z_hz / (1.0 + b_hz_x);      /* C_HZXLX */
-      cell[6 * n + k] = ns_coef1(b_hz_y);                  /* C_HZY */
-      cell[7 * n + k] = u_hz / z_hz / (1.0 + b_hz_y);      /* C_HZYLY */
-      const double z_ex = sqrt(mu0 / e_ex), n_ex = sqrt(e_ex / eps0);
-      const double u_ex = sin(w_s * 0.5) / sin(k_s * n_ex * 0.5);
-      cell[k] = ns_coef1(b_ex_y);                          /* C_EX */
-      cell[n + k] = u_ex * z_ex / (1.0 + b_ex_y);          /* C_EXLY */
-      const double z_ey = sqrt(mu0 / e_ey), n_ey = sqrt(e_ey / eps0);
-      const double u_ey = sin(w_s * 0.5) / sin(k_s * n_ey * 0.5);
-      cell[2 * n + k] = ns_coef1(b_ey_x);                  /* C_EY */
-      cell[3 * n + k] = u_ey * z_ey / (1.0 + b_ey_x);      /* C_EYLX */
-      cell[8 * n + k] = ns_wave_factor(e_ex, eps0, w_s, k_s);
-      cell[9 * n + k] = ns_wave_factor(e_ey, eps0, w_s, k_s);
-    }
+  const double *sig[4] = {t, t + nx, t + 2 * nx, t + 2 * nx + ny};
+  for (int i = 0; i < nx; i++) {
+    t[i] = sig_max * field_sigmaX(i, 0);
+    t[nx + i] = sig_max * field_sigmaX(i + 0.5, 0);
   }
-}
-
-/* nsFdtdTM.c:226-306 / nsFdtdTE.c:100-181 and field.c:155-177: the per-cell
-   coefficients of the NS solvers from the eps maps the device filled (TM EPS_EZ,
-   EPS_HX, EPS_HY; TE EPS_EX, EPS_EY, EPS_HZ), each formed with the reference's
-   expression and operation order */
-static int build_ns_coefs(int kind, fdtd_grid *g)
-{
-  const int nx = N_PX, ny = N_PY;
-  const size_t n = (size_t)nx * ny;
-  const int nmaps = is_tm(kind) ? 5 : 10;
-  double *eps = (double *)malloc(3 * n * sizeof(double)), *cell = (double *)malloc(nmaps * n * sizeof(double));
-  if (!eps || !cell) {
-    free(eps);
-    free(cell);
-    return FDTD_ENOMEM;
+  for (int j = 0; j < ny; j++) {
+    t[2 * nx + j] = sig_max * field_sigmaY(0, j);
+    t[2 * nx + ny + j] = sig_max * field_sigmaY(0, j + 0.5);
   }
-  int rc = FDTD_OK;
-  for (int q = 0; q < 3 && rc == FDTD_OK; q++) rc = fdtd_hip_grid_get_eps(g, q, eps + q * n);
-  const double R = 1.0e-8, M = 2.0, eps0 = 1.0, C = field_getLightSpeed(), mu0 = field_getMu0();
-  const double sig_max = -(M + 1.0) * eps0 * C / N_PML * log(R);
-  const double w_s = field_getOmega(), k_s = field_getK();
-  if (rc == FDTD_OK && !is_tm(kind)) ns_te_cells(eps, cell, n);
-  for (int i = 0; i < nx && rc == FDTD_OK && is_tm(kind); i++) {
-    const double b_ez_x = ns_beta(sig_max * field_sigmaX(i, 0) / (2 * eps0));
-    const double b_hy_x = ns_beta(sig_max * field_sigmaX(i + 0.5, 0) / (2 * eps0));
-    for (int j = 0; j < ny; j++) {
-      const size_t k = (size_t)i * ny + j;
-      const double b_hx_y = ns_beta(sig_max * field_sigmaY(0, j + 0.5) / (2 * eps0));
-      const double e_ez = eps[k], e_hx = eps[n + k], e_hy = eps[2 * n + k];
-      const double z_ez = sqrt(mu0 / e_ez), n_ez = sqrt(e_ez / eps0);
-      const double u_ez = sin(w_s * 0.5) / sin(k_s * n_ez * 0.5);
-      cell[k] = u_ez * z_ez / (1 + b_ez_x);          /* C_EZXLX */
-      cell[n + k] = u_ez * z_ez / (1.0 + b_ez_x);    /* C_EZYLY: b_ez_x, as nsFdtdTM.c:282 has it */
-      const double z_hx = sqrt(mu0 / e_hx), n_hx = sqrt(e_hx / eps0);
-      const double u_hx = sin(w_s * 0.5) / sin(k_s * n_hx * 0.5);
-      cell[2 * n + k] = u_hx / z_hx / (1.0 + b_hx_y);  /* C_HXLY */
-      const double z_hy = sqrt(mu0 / e_hy), n_hy = sqrt(e_hy / eps0);
-      const double u_hy = sin(w_s * 0.5) / sin(k_s * n_hy * 0.5);
-      cell[3 * n + k] = u_hy / z_hy / (1.0 + b_hy_x);  /* C_HYLX */
-      cell[4 * n + k] = ns_wave_factor(e_ez, eps0, w_s, k_s);
-    }
-  }
+  const double k_s = field_getK();
   const double r = 1.0 / 6.0 + k_s * k_s / 180.0 - pow(k_s, 4) / 23040;  /* nsFdtdTM.c:117, nsFdtdTE.c:255 */
-  if (rc == FDTD_OK) rc = fdtd_hip_grid_set_ns_coefs(g, cell, r / 2.0);
-  free(eps);
-  free(cell);
+  const int rc = fdtd_hip_grid_form_ns_coefs(g, sig, field_getOmega(), k_s, r / 2.0);
+  free(t);
   return rc;
 }
 
@@ -382,7 +312,7 @@ int solver_make_grid(int kind, int precision, int ntff_time, int T, int R, fdtd_
   build_coefs(kind, g);
   if ((rc = fdtd_hip_grid_fill_eps(g, models_getState())) == FDTD_OK && precision == FDTD_FP32)
     rc = fdtd_hip_grid_set_blocking(g, T > 0 ? T : 4, R);
-  if (rc == FDTD_OK && is_ns(kind)) rc = build_ns_coefs(kind, g);
+  if (rc == FDTD_OK && is_ns(kind)) rc = build_ns_coefs(g);
   if (rc != FDTD_OK) {
     fdtd_hip_grid_destroy(g);
     return rc;
