@@ -710,7 +710,7 @@ __global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Co
 // on the step (a = 0.5 + ts - dE for E, ts - (dH - 1) for H): the bins and
 // weights of the reference's calc() (ntffTM.c:279-288, mpiTM_UPML.c:994-1036).
 //
-// The host sorts the samples of each (angle, target array) by offset d and cuts
+// k_bin_records sorts the samples of each (angle, target array) by offset d and cuts
 // the sorted list into parts of at most NTFF_GRP x NTFF_RUN samples spanning at
 // most NTFF_WIN offsets, one workgroup each.  A workgroup is NTFF_GRP groups of
 // NS >= n lanes; group g takes a contiguous run of the part's sorted samples
@@ -1485,29 +1485,12 @@ static void build_contour(fdtd_grid *g)
   ct.total = off;
 }
 
-// retarded-time shift of every (angle, contour cell), formed on the host with
-// the reference's own arithmetic: direct per cell for the MPI solvers
-// (mpiTM_UPML.c:894), accumulated along each side for the plain ones (ntffTM.c:329-334)
 // The reference forms the angle as ang*M_PI/180.0 in the MPI NTFF, the far
 // field and ntffTE_TimeTranslate (angle table A), but as ang*ToRad with
 // ToRad = M_PI/180.0 in ntffTM_TimeCalc / ntffTE_TimeCalc / ntffTM_TimeTranslate
 // (table B, ntffTM.c:314-318, ntffTE.c:89-92, ntffTM.c:169-173); the two differ in the last bit.
-// the per-(angle, contour cell) time shifts (tab, only when with_tab) and the
-// angle tables
-static void build_time_shift(const fdtd_grid *g, std::vector<double> &tab, std::vector<double> &mn, std::vector<double> &mx,
-                             std::vector<double> &ca, std::vector<double> &sa, std::vector<double> &cb, std::vector<double> &sb,
-                             bool with_tab = true)
+static void build_angles(double *ca, double *sa, double *cb, double *sb)
 {
-  const fdtd_grid_desc &d = g->d;
-  const Contour &ct = g->ct;
-  const bool mpi = d.flavour == FDTD_FLAVOUR_MPI;
-  tab.assign(with_tab ? (size_t)360 * ct.total : 0, 0.0);
-  mn.assign(360, 0.0);
-  mx.assign(360, 0.0);
-  ca.resize(360);
-  sa.resize(360);
-  cb.resize(360);
-  sb.resize(360);
   const double ToRad = M_PI / 180.0;
   for (int ang = 0; ang < 360; ang++) {
     const double radA = ang * M_PI / 180.0, radB = ang * ToRad;
@@ -1515,100 +1498,205 @@ static void build_time_shift(const fdtd_grid *g, std::vector<double> &tab, std::
     sa[ang] = sin(radA);
     cb[ang] = cos(radB);
     sb[ang] = sin(radB);
-    if (!with_tab) continue;
-    const double r1x = mpi ? ca[ang] : cb[ang], r1y = mpi ? sa[ang] : sb[ang];
-    double *t = &tab[(size_t)ang * ct.total];
-    for (int q = 0; q < 4; q++) {
-      const Seg &s = ct.s[q];
-      if (mpi) {
-        for (int c = 0; c < s.n; c++) {
-          const double r2x = s.r2x0 + c * s.dr2x, r2y = s.r2y0 + c * s.dr2y;
-          t[s.off + c] = -(r1x * r2x + r1y * r2y) / d.c0 + d.rf_per_c;
-        }
-      } else {
-        const double r1x_per_c = r1x / d.c0, r1y_per_c = r1y / d.c0;
-        double ts = -(r1x_per_c * s.r2x0 + r1y_per_c * s.r2y0) + d.rf_per_c;
-        const double step = (q == 0 || q == 2) ? r1x_per_c : r1y_per_c;
-        for (int c = 0; c < s.n; c++) {
-          t[s.off + c] = ts;
-          ts -= step;
-        }
-      }
-    }
-    double lo = 1e300, hi = -1e300;
-    for (int p = 0; p < ct.total; p++) {
-      lo = std::min(lo, t[p]);
-      hi = std::max(hi, t[p]);
-    }
-    mn[ang] = ct.total ? lo : 0.0;
-    mx[ang] = ct.total ? hi : 0.0;
   }
 }
 
-// The records of k_ntff_bin: the samples of each (angle, target array) sorted by
-// offset d, cut into parts of at most NTFF_GRP x NTFF_RUN samples and NTFF_WIN
-// offsets, each part split into NTFF_GRP contiguous runs stored [iteration][group].
-static int build_bin_groups(fdtd_grid *g, const std::vector<double> &tab)
+// Retarded-time shift of every (angle, contour cell), with the reference's own
+// arithmetic: direct per cell for the MPI solvers (mpiTM_UPML.c:894), accumulated along
+// each side for the plain ones (ntffTM.c:329-334).  One thread per angle and side.
+__global__ __launch_bounds__(64) void k_time_shift(Contour ct, int mpi, const double *cs, const double *sn, double c0,
+                                                   double rf, double *ts)
 {
-  const Contour &ct = g->ct;
-  const int P = ct.total;
+  const int id = blockIdx.x * 64 + threadIdx.x, ang = id >> 2;
+  if (ang >= 360) return;
+  const Seg &s = ct.s[id & 3];
+  const double r1x = cs[ang], r1y = sn[ang];
+  double *t = ts + (size_t)ang * ct.total + s.off;
+  if (mpi) {
+    for (int c = 0; c < s.n; c++) {
+      const double r2x = s.r2x0 + c * s.dr2x, r2y = s.r2y0 + c * s.dr2y;
+      t[c] = -(r1x * r2x + r1y * r2y) / c0 + rf;
+    }
+  } else {
+    const double r1x_per_c = r1x / c0, r1y_per_c = r1y / c0;
+    double v = -(r1x_per_c * s.r2x0 + r1y_per_c * s.r2y0) + rf;
+    const double step = (id & 1) ? r1y_per_c : r1x_per_c;
+    for (int c = 0; c < s.n; c++) {
+      t[c] = v;
+      v -= step;
+    }
+  }
+}
+
+// the shifts into ts[360][total] (device)
+static int time_shifts(fdtd_grid *g, double *ts)
+{
+  const bool mpi = g->d.flavour == FDTD_FLAVOUR_MPI;
+  hipLaunchKernelGGL(k_time_shift, dim3(360 * 4 / 64 + 1), dim3(64), 0, 0, g->ct, mpi ? 1 : 0, mpi ? g->cosA : g->cosB,
+                     mpi ? g->sinA : g->sinB, g->d.c0, g->d.rf_per_c, ts);
+  HIPCHK(hipGetLastError());
+  return FDTD_OK;
+}
+
+// The records of k_ntff_bin, one workgroup per (angle, target array): a counting sort
+// of the array's samples by offset d, BIN_SORT offsets at a time, the sorted list cut
+// into parts of at most NTFF_GRP x NTFF_RUN samples that do not cross a multiple of
+// NTFF_WIN offsets, each part split into NTFF_GRP contiguous runs stored
+// [iteration][group].  Records the host had filled with -1 pad the runs.  Sorted on one
+// host core and uploaded, the 3 million samples of the 1056 x 1056 grid's contour took
+// 40 ms of a 48 ms run of 4000 steps.
+#define BIN_SORT (8 * NTFF_WIN)
+__global__ __launch_bounds__(256) void k_bin_records(const double *ts, Contour ct, int nb, BinPart *parts, BinRec *rec, int *ctr)
+{
+  __shared__ int offs[BIN_SORT + 1], cur[BIN_SORT], sums[256], lim[2], blk[BIN_SORT / NTFF_WIN];
+  const int ang = blockIdx.x, arr = blockIdx.y, P = ct.total, tid = threadIdx.x;
+  const double *t = ts + (size_t)ang * P;
+  // sample e: E of cell e, or H of cell e - P; its offset and tap fraction if it goes to this array
+  auto sample = [&](int e, int &d, double &a) -> bool {
+    const int hh = e >= P, p = hh ? e - P : e;
+    int q = 0;
+    while (q < 3 && p >= ct.s[q + 1].off) q++;
+    if ((hh ? ct.s[q].wa : ct.s[q].ua) != arr) return false;
+    const double v = t[p];
+    d = hh ? (int)floor(v) + 1 : (int)floor(v + 0.5);
+    a = hh ? v - (double)(d - 1) : (0.5 + v) - (double)d;
+    return true;
+  };
+  if (tid == 0) {
+    lim[0] = INT_MAX;
+    lim[1] = INT_MIN;
+  }
+  __syncthreads();
+  int lo = INT_MAX, hi = INT_MIN, d = 0;
+  double a = 0.0;
+  for (int e = tid; e < 2 * P; e += 256)
+    if (sample(e, d, a)) {
+      lo = min(lo, d);
+      hi = max(hi, d);
+    }
+  atomicMin(&lim[0], lo);
+  atomicMax(&lim[1], hi);
+  __syncthreads();
+  const int dmin = lim[0], dmax = lim[1];
+  if (dmin > dmax) return;
+  for (long w0 = dmin; w0 <= dmax; w0 += BIN_SORT) {
+    for (int q = tid; q < BIN_SORT; q += 256) cur[q] = 0;
+    __syncthreads();
+    for (int e = tid; e < 2 * P; e += 256)
+      if (sample(e, d, a) && d >= w0 && d < w0 + BIN_SORT) atomicAdd(&cur[d - w0], 1);
+    __syncthreads();
+    // exclusive scan: BIN_SORT / 256 offsets per thread, then the threads' sums
+    constexpr int PT = BIN_SORT / 256;
+    int s = 0;
+    for (int q = 0; q < PT; q++) s += cur[tid * PT + q];
+    sums[tid] = s;
+    __syncthreads();
+    if (tid == 0) {
+      int acc = 0;
+      for (int q = 0; q < 256; q++) {
+        const int v = sums[q];
+        sums[q] = acc;
+        acc += v;
+      }
+      offs[BIN_SORT] = acc;
+    }
+    __syncthreads();
+    s = sums[tid];
+    for (int q = 0; q < PT; q++) {
+      offs[tid * PT + q] = s;
+      s += cur[tid * PT + q];
+    }
+    __syncthreads();
+    for (int q = tid; q < BIN_SORT; q += 256) cur[q] = offs[q];
+    // the parts of every NTFF_WIN offsets
+    constexpr int MAXS = NTFF_GRP * NTFF_RUN;
+    if (tid == 0) {
+      int n = 0;
+      for (int b = 0; b < BIN_SORT / NTFF_WIN; b++) {
+        blk[b] = n;
+        n += (offs[(b + 1) * NTFF_WIN] - offs[b * NTFF_WIN] + MAXS - 1) / MAXS;
+      }
+      const int base = atomicAdd(&ctr[0], n);
+      for (int b = 0; b < BIN_SORT / NTFF_WIN; b++) blk[b] += base;
+    }
+    __syncthreads();
+    for (int b = 0; b < BIN_SORT / NTFF_WIN; b++) {
+      const int x0 = offs[b * NTFF_WIN], x1 = offs[(b + 1) * NTFF_WIN];
+      for (int q = tid; x0 + q * MAXS < x1; q += 256) {
+        const int y0 = x0 + q * MAXS, y1 = min(x1, y0 + MAXS);
+        // the offset that sorted sample y lies on: the last one whose samples begin at or before y
+        auto at = [&](int y) {
+          int l = b * NTFF_WIN, h = (b + 1) * NTFF_WIN - 1;
+          while (l < h) {
+            const int m = (l + h + 1) >> 1;
+            if (offs[m] <= y) l = m;
+            else h = m - 1;
+          }
+          return l;
+        };
+        const int l = at(y0), h = at(y1 - 1);
+        BinPart W;
+        W.per = (y1 - y0 + NTFF_GRP - 1) / NTFF_GRP;
+        W.rec0 = atomicAdd(&ctr[1], W.per * NTFF_GRP);
+        W.dlo = (int)w0 + l;
+        W.nd = h - l + 1;
+        W.row = ang;
+        W.arr = arr;
+        parts[blk[b] + q] = W;
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int e = tid; e < 2 * P; e += 256)
+      if (sample(e, d, a) && d >= w0 && d < w0 + BIN_SORT) {
+        const int o = (int)(d - w0), b = o / NTFF_WIN, x = atomicAdd(&cur[o], 1) - offs[b * NTFF_WIN];
+        const BinPart &W = parts[blk[b] + x / MAXS];
+        const int i = x % MAXS;
+        rec[(size_t)W.rec0 + (size_t)(i % W.per) * NTFF_GRP + i / W.per] = BinRec{e * nb, d - W.dlo, a};
+      }
+    __syncthreads();
+  }
+}
+
+static int build_bin_groups(fdtd_grid *g)
+{
+  const int P = g->ct.total;
   // a record addresses its sample's first step directly: cell p of E at p * nb,
   // of H at (P + p) * nb (the sample buffer holds E then H, nb steps per cell)
   const int nb = g->nbuf;
   if ((size_t)2 * P * nb > (size_t)INT_MAX) return fdtd_fail(FDTD_ENOMEM, "NTFF contour of %d cells too long", P);
-  std::vector<BinPart> parts;
-  std::vector<BinRec> rec;
-  std::vector<int> side(P);
+  // parts: full ones, and one that is not per NTFF_WIN offsets an array's samples reach (a
+  // shift spans at most the contour's diagonal over c0 on top of its rounding)
+  double lo = 0, hi = 0;
   for (int q = 0; q < 4; q++)
-    for (int c = 0; c < ct.s[q].n; c++) side[ct.s[q].off + c] = q;
-  struct Smp {
-    int d, p;
-    double a;
-  };
-  std::vector<Smp> by[3];
-  for (int ang = 0; ang < 360; ang++) {
-    const double *ts = &tab[(size_t)ang * P];
-    for (int arr = 0; arr < 3; arr++) by[arr].clear();
-    for (int p = 0; p < P; p++) {
-      const Seg &sg = ct.s[side[p]];
-      const int dE = (int)floor(ts[p] + 0.5), dH = (int)floor(ts[p]) + 1;
-      by[sg.ua].push_back({dE, p * nb, (0.5 + ts[p]) - (double)dE});
-      by[sg.wa].push_back({dH, (P + p) * nb, ts[p] - (double)(dH - 1)});
+    for (int e = 0; e < 2; e++) {
+      const Seg &s = g->ct.s[q];
+      const double x = s.r2x0 + (e ? (s.n - 1) * s.dr2x : 0.0), y = s.r2y0 + (e ? (s.n - 1) * s.dr2y : 0.0);
+      const double r = s.n ? sqrt(x * x + y * y) / g->d.c0 : 0.0;
+      hi = std::max(hi, r);
+      lo = std::min(lo, -r);
     }
-    for (int arr = 0; arr < 3; arr++) {
-      std::vector<Smp> &v = by[arr];
-      std::stable_sort(v.begin(), v.end(), [](const Smp &x, const Smp &y) { return x.d < y.d; });
-      size_t x0 = 0;
-      while (x0 < v.size()) {
-        const int dlo = v[x0].d;
-        size_t x1 = x0;
-        while (x1 < v.size() && x1 - x0 < NTFF_GRP * NTFF_RUN && v[x1].d < dlo + NTFF_WIN) x1++;
-        BinPart W;
-        W.rec0 = (int)rec.size();
-        W.dlo = dlo;
-        W.nd = v[x1 - 1].d - dlo + 1;
-        W.row = ang;
-        W.arr = arr;
-        const int cnt = (int)(x1 - x0);
-        W.per = (cnt + NTFF_GRP - 1) / NTFF_GRP;
-        rec.resize(rec.size() + (size_t)W.per * NTFF_GRP, BinRec{-1, 0, 0.0});
-        for (int t = 0; t < NTFF_GRP; t++)
-          for (int i = 0; i < W.per; i++) {
-            const size_t x = x0 + (size_t)t * W.per + i;
-            if (x >= x1) break;
-            rec[(size_t)W.rec0 + (size_t)i * NTFF_GRP + t] = BinRec{v[x].p, v[x].d - dlo, v[x].a};
-          }
-        parts.push_back(W);
-        x0 = x1;
-      }
-    }
-  }
-  if (rec.size() > (size_t)INT_MAX) return fdtd_fail(FDTD_ENOMEM, "NTFF binning records exceed 2^31");
-  g->nparts = (int)parts.size();
-  HIPCHK(dev_malloc(&g->binPart, std::max<size_t>(1, parts.size()) * sizeof(BinPart)));
-  HIPCHK(dev_malloc(&g->binRec, std::max<size_t>(1, rec.size()) * sizeof(BinRec)));
-  if (!parts.empty()) HIPCHK(hipMemcpy(g->binPart, parts.data(), parts.size() * sizeof(BinPart), hipMemcpyHostToDevice));
-  if (!rec.empty()) HIPCHK(hipMemcpy(g->binRec, rec.data(), rec.size() * sizeof(BinRec), hipMemcpyHostToDevice));
+  const size_t win = (size_t)((hi - lo + 8) / NTFF_WIN) + 2;
+  const size_t maxp = (size_t)360 * 2 * P / (NTFF_GRP * NTFF_RUN) + (size_t)360 * 3 * win;
+  const size_t maxr = (size_t)360 * 2 * P + maxp * NTFF_GRP;
+  if (maxr > (size_t)INT_MAX) return fdtd_fail(FDTD_ENOMEM, "NTFF binning records exceed 2^31");
+  HIPCHK(dev_malloc(&g->binPart, maxp * sizeof(BinPart)));
+  HIPCHK(dev_malloc(&g->binRec, maxr * sizeof(BinRec)));
+  HIPCHK(hipMemsetAsync(g->binRec, 0xff, maxr * sizeof(BinRec), 0));
+  double *ts = nullptr;
+  int *ctr = nullptr;
+  HIPCHK(dev_malloc(&ts, (size_t)360 * P * sizeof(double)));
+  HIPCHK(dev_malloc(&ctr, 2 * sizeof(int)));
+  HIPCHK(hipMemsetAsync(ctr, 0, 2 * sizeof(int), 0));
+  int rc = time_shifts(g, ts);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_bin_records, dim3(360, 3), dim3(256), 0, 0, ts, g->ct, nb, g->binPart, g->binRec, ctr);
+  HIPCHK(hipGetLastError());
+  int n[2] = {0, 0};
+  HIPCHK(hipMemcpy(n, ctr, sizeof n, hipMemcpyDeviceToHost));
+  g->nparts = n[0];
+  HIPCHK(dev_free(ts));
+  HIPCHK(dev_free(ctr));
   return FDTD_OK;
 }
 
@@ -1824,8 +1912,8 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
     HIPCHK(hipMemset(g->ntb[a], 0, g->ntn * sizeof(double2)));
     g->nt[a] = g->ntb[a] + NT_GUARD;
   }
-  std::vector<double> tab, mn, mx, ca, sa, cb, sb;
-  build_time_shift(g, tab, mn, mx, ca, sa, cb, sb, d->ntff_time != 0);
+  double ca[360], sa[360], cb[360], sb[360];
+  build_angles(ca, sa, cb, sb);
   const int P = std::max(1, g->ct.total);
   // blocked paths bin a whole block of steps at once: sample buffers for as many
   const bool upml = d->flavour == FDTD_FLAVOUR_MPI || d->flavour == FDTD_FLAVOUR_PLAIN;
@@ -1834,18 +1922,18 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
   // (the binning's records address both from cE)
   HIPCHK(dev_malloc(&g->cE, (size_t)2 * g->nbuf * P * sizeof(double2)));
   g->cH = g->cE + (size_t)g->nbuf * P;
-  if (d->ntff_time && g->ct.total > 0) {
-    int rc = build_bin_groups(g, tab);
-    if (rc) return rc;
-  }
   HIPCHK(dev_malloc(&g->cosA, 360 * sizeof(double)));
   HIPCHK(dev_malloc(&g->sinA, 360 * sizeof(double)));
-  HIPCHK(hipMemcpy(g->cosA, ca.data(), 360 * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(g->sinA, sa.data(), 360 * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(g->cosA, ca, 360 * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(g->sinA, sa, 360 * sizeof(double), hipMemcpyHostToDevice));
   HIPCHK(dev_malloc(&g->cosB, 360 * sizeof(double)));
   HIPCHK(dev_malloc(&g->sinB, 360 * sizeof(double)));
-  HIPCHK(hipMemcpy(g->cosB, cb.data(), 360 * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(g->sinB, sb.data(), 360 * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(g->cosB, cb, 360 * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(g->sinB, sb, 360 * sizeof(double), hipMemcpyHostToDevice));
+  if (d->ntff_time && g->ct.total > 0) {
+    int rc = build_bin_groups(g);
+    if (rc) return rc;
+  }
   // 1/(4 pi c R), R = 1e6, applied per step by the MPI solvers (mpiTM_UPML.c:852-854)
   g->coef = 1.0 / (4 * M_PI * d->c0 * 1.0e6);
   HIPCHK(dev_malloc(&g->ffout, 360 * sizeof(double2)));
@@ -2593,10 +2681,8 @@ extern "C" int fdtd_hip_grid_set_dft(fdtd_grid *g, const double *omega, int nf)
   HIPCHK(hipMemset(g->dftE, 0, (size_t)nf * P * sizeof(double2)));
   HIPCHK(hipMemset(g->dftH, 0, (size_t)nf * P * sizeof(double2)));
   HIPCHK(dev_malloc(&g->dftOut, (size_t)nf * 3 * 360 * sizeof(double2)));
-  std::vector<double> tab, mn, mx, ca, sa, cb, sb;
-  build_time_shift(g, tab, mn, mx, ca, sa, cb, sb);
-  HIPCHK(dev_malloc(&g->dftTs, tab.size() * sizeof(double)));
-  HIPCHK(hipMemcpy(g->dftTs, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(dev_malloc(&g->dftTs, (size_t)360 * P * sizeof(double)));
+  if ((rc = time_shifts(g, g->dftTs))) return rc;
   g->nf = nf;
   // the FP32 fused kernel samples the contour after every inner step
   if (g->fs && !g->ctrSet) {
