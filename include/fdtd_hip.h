@@ -209,8 +209,8 @@ int fdtd_hip_grid_sync(fdtd_grid *g);
 int fdtd_hip_grid_set_blocking(fdtd_grid *g, int T, int R);
 int fdtd_hip_grid_get_blocking(const fdtd_grid *g, int *T, int *R);
 /* FP32 grids: how a block's UPML and interior tiles are launched.  AUTO picks
- * SPLIT for large grids (over 4096 interior workgroups, 8 per UPML one), else
- * MERGED; MERGED is one launch of both
+ * MERGED for small grids (plain TE: TWO_STREAMS_P16) and SPLIT_P16 from 0.8 (TE), 1
+ * (plain TM) or 4 (MPI TM) million cells; MERGED is one launch of both
  * (one register budget, the UPML body's); SPLIT is two launches in a row, each
  * at its own occupancy; TWO_STREAMS runs the two launches side by side on two
  * streams. */

@@ -1687,24 +1687,44 @@ static int update_wave(FastState *s, const fdtd_step_params &p)
   return FDTD_OK;
 }
 
+// The launch shape of FAST_LAUNCH_AUTO: one merged launch while the tiles leave the
+// chip partly idle, the two kinds apart with 8- and 16-wavefront tiles once each
+// fills it; the plain TE body, which spills at the merged kernel's budget, beside each
+// other on two streams instead.  The lines lie between the sizes timed (8-step blocks,
+// R = 16, us; merged / SPLIT_P16 / TWO_STREAMS_P16 on 500 x 400, 1056 x 1056 and
+// 2000 x 1500 cells): MPI TM 24/36/44, 34/43/54, 59/62/74; MPI TE 25/39/45, 53/48/57,
+// 100/72/83; plain TM 34/47/43, 51/50/58, 76/69/79; plain TE 60/66/46, 91/65/72,
+// 148/86/95.  The former two-launch shape of large grids (SPLIT, 4-wavefront tiles) took
+// 71, 93, 88 and 137 on 2000 x 1500.
+static int auto_shape(const FastState *s)
+{
+  const size_t cells = (size_t)s->h.NPX * s->h.NPY;
+  const bool tm = s->d.mode == FDTD_MODE_TM, mpi = s->d.flavour == FDTD_FLAVOUR_MPI;
+  const size_t line = tm ? (mpi ? (size_t)4 << 20 : (size_t)1 << 20) : (size_t)3 << 18;
+  if (cells >= line) return FAST_LAUNCH_SPLIT_P16;
+  return tm || mpi ? FAST_LAUNCH_MERGED : FAST_LAUNCH_TWO_STREAMS_P16;
+}
+
 int fast_state_flush(FastState *s)
 {
   if (s->pending == 0) return FDTD_OK;
   int rc;
   const int Tsave = s->T;
+  const int mode = s->lmode == FAST_LAUNCH_AUTO ? auto_shape(s) : s->lmode;
   // the UPML bodies of the *_PML8, *_W8 and *_P16 shapes cover the wide tiles
   {
-    const int lm = s->lmode;
+    const int lm = mode;
     const bool wide = !s->batch && (lm == FAST_LAUNCH_SPLIT_PML8 || lm == FAST_LAUNCH_TWO_STREAMS_PML8 ||
                                     lm == FAST_LAUNCH_SPLIT_W8 || lm == FAST_LAUNCH_TWO_STREAMS_W8 ||
                                     lm == FAST_LAUNCH_SPLIT_P16 || lm == FAST_LAUNCH_TWO_STREAMS_P16);
     s->upmlRows = wide ? FAST_UPML_ROWS_WIDE : FAST_UPML_ROWS;
     // R = 18 and 20 (72- and 80-row interior tiles) exist only as 8 wavefronts of 9 and 10 rows
-    const bool i8 = lm == FAST_LAUNCH_SPLIT_W8 || lm == FAST_LAUNCH_TWO_STREAMS_W8 || lm == FAST_LAUNCH_SPLIT_P16 ||
-                    lm == FAST_LAUNCH_TWO_STREAMS_P16;
+    const int set = s->lmode;  // AUTO, whose choice depends on the grid, does not take them
+    const bool i8 = set == FAST_LAUNCH_SPLIT_W8 || set == FAST_LAUNCH_TWO_STREAMS_W8 || set == FAST_LAUNCH_SPLIT_P16 ||
+                    set == FAST_LAUNCH_TWO_STREAMS_P16;
     if ((s->R == 18 || s->R == 20) && !i8)
       return fdtd_fail(FDTD_EINVAL, "R=%d needs a launch shape with 8-wavefront interior tiles (*_W8, *_P16), not %d",
-                       s->R, lm);
+                       s->R, set);
   }
   // a partial block runs with T = pending; the tiles of the full depth stay valid
   // for any smaller depth, so only the block depth passed to the kernel changes
@@ -1736,11 +1756,6 @@ int fast_state_flush(FastState *s)
   memcpy(a.qb[0], s->qpml, sizeof a.qb[0]);
   memcpy(a.qb[1], s->qint, sizeof a.qb[1]);
   const int nbp = 8 * ((s->n_pml + 7) / 8), nbi = 8 * ((s->n_int + 7) / 8);
-  int mode = s->lmode;
-  if (mode == FAST_LAUNCH_AUTO)
-    // large grid: interior and UPML tiles as two launches, each at its own
-    // occupancy (the interior body's register budget is below the UPML body's)
-    mode = (nbi >= 8 * nbp && nbi > 4096) ? FAST_LAUNCH_SPLIT : FAST_LAUNCH_MERGED;
   s->lmode_last = mode;
   // the interior (UPML) tiles: those off the contour with the plain kind, those
   // on it with the sampling kind (without samples, all of a list is off it)
