@@ -46,7 +46,8 @@
 // A strip: core rows [r0, r1) x columns [j0, j1) written; lane 0's first column
 // bj, first input row b0, last input row bl (array coordinates, ring included).
 struct StreamStrip {
-  int j0, j1, bj, r0, r1, b0, bl, kind, smp, pad[7];
+  int j0, j1, bj, r0, r1, b0, bl, kind;
+  int smp, s0, s1, pad[5];  // contour sides through the strip (a bit each), rows with their samples
 };
 
 struct StreamSide {
@@ -105,9 +106,10 @@ __host__ __device__ constexpr int stream_lds_i(int mode, int C, int S) { return 
 // PF: rows fetched ahead of the one that enters the first stage (a row's turn is
 // shorter than a load's latency)
 template <int MODE, int FLAV, int PML, int C, int S, int PF>
-__device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStrip t, D2 *lv, double *li)
+__device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStrip t, D2 *lv, double *li, D2 *ls)
 {
   constexpr bool TM = MODE == FDTD_MODE_TM, MPI = FLAV == FDTD_FLAVOUR_MPI;
+  static_assert(S == 2 && STREAM_T / S > 2, "the sampling of the first wavefront's steps");
   constexpr int K = STREAM_T / S, NS = (MPI ? S + 1 : S + 2) + PF;
   // values of a cell.  Interior TM: E Hx Hy, TE: Ex Ey Hz.
   // Frame TM: E J D Mx Bx My By, TE: Ex Ey Bz Mz Jx Dx Jy Dy
@@ -405,33 +407,53 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
     if (!PML) return V[q][v][c];
     return mul(c2, V[q][TM ? (v == 1 ? 4 : 6) : 2][0]);
   };
-  // contour samples of the finished row r in slot q after step entry st
-  auto sample = [&](int q, int r, int st) {
-    if (r < t.r0 || r >= t.r1) return;
+  // Contour samples of row r after step entry st, its values from val(v, c): TM E Hx Hy,
+  // TE Ex Ey Hz.  The first wavefront stores none itself: it waits for its loads, and a
+  // store among them would be waited for as well (rows of 2.1 us instead of 0.8).  It
+  // leaves the row of its first step in ls for the second wavefront, and every wavefront
+  // samples its predecessor's last step from the row it takes.
+  auto sample = [&](int r, int st, auto val) {
     CAS(StreamArgs) R = rare_args();
     const int tot = R->ctot;
     D2 *base = R->csamp + (size_t)(st - 1) * 3 * tot;
 #pragma unroll 1
-    for (int sd = 0; sd < 4; sd++) {
-      const CAS_(StreamSide) &g = R->side[sd];
-      if (g.n <= 0) continue;
+    for (int m = t.smp; m; m &= m - 1) {
+      const CAS_(StreamSide) &g = R->side[__builtin_ctz(m)];
+      const int lo = g.lo, fi = g.fi, off = g.off;
+      if (g.horiz ? r < lo || r >= lo + g.n : r != fi && r != fi - 1) continue;
 #pragma unroll
       for (int c = 0; c < C; c++) {
         const int j = col + c;
         if (j < t.j0 || j >= t.j1) continue;
-        const D2 e = g.ef ? V[q][TM ? 0 : 1][c] : V[q][0][c];
-        const D2 h = TM ? (g.hf == 1 ? hval(q, 1, c) : hval(q, 2, c)) : hval(q, 2, c);
         const int x = g.horiz ? j : r, y = g.horiz ? r : j;  // across, along the side
-        if (y < g.lo || y >= g.lo + g.n) continue;
-        const int p = g.off + (y - g.lo);
-        if (x == g.fi) {
-          base[p] = mul(g.es, e);
+        if (y < lo || y >= lo + g.n) continue;
+        const D2 h = TM && g.hf == 1 ? val(1, c) : val(2, c);
+        const int p = off + (y - lo);
+        if (x == fi) {
+          base[p] = mul(g.es, TM || !g.ef ? val(0, c) : val(1, c));
           base[tot + p] = h;
-        } else if (x == g.fi - 1) {
+        } else if (x == fi - 1) {
           base[2 * tot + p] = h;
         }
       }
     }
+  };
+  const int s1 = a.csamp ? t.s1 : t.s0;
+  auto sampled = [&](int r) { return r >= t.s0 && r < s1; };
+  // values of the row in slot q as sample takes them
+  auto field = [&](int q) {
+    return [&, q](int v, int c) -> D2 { return TM ? (v ? hval(q, v, c) : V[q][0][c]) : (v < 2 ? V[q][v][c] : hval(q, 2, c)); };
+  };
+  auto leave = [&](int q, int p) {
+    D2 *o = ls + p * (3 * C * 64) + lane;
+    auto val = field(q);
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+      for (int v = 0; v < 3; v++) o[(v * C + c) * 64] = val(v, c);
+  };
+  auto left = [&](int p) {
+    return [&, p](int v, int c) -> D2 { return ls[p * (3 * C * 64) + (v * C + c) * 64 + lane]; };
   };
   auto store = [&](int q, int r) {
     if (r < t.r0 || r >= t.r1) return;
@@ -495,7 +517,6 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
   const int row0 = t.b0 - w * (S + 2);
   const int nit = (t.r1 - t.b0) + S + (K - 1) * (S + 2);
   const int st0 = w * S;
-  const bool smp = t.smp && a.csamp;
   // A copy of the row loop for the first, the last and the other wavefronts: with
   // the loads, the stores and the LDS reads of a row in one copy, the compiler waits
   // for every outstanding load wherever the branches join.
@@ -519,7 +540,11 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
         if (first) settle(u, n);
         else flag(u, n);
         if (first) load((u + PF) % NS, n + PF);
-        else take((u + 1) % NS, (it + 1) & 1);
+        else {
+          take((u + 1) % NS, (it + 1) & 1);
+          if (RARE(sampled(n + 1)) && st0 <= a.T) sample(n + 1, st0, field((u + 1) % NS));
+          if (w == 1 && RARE(sampled(n + S))) sample(n + S, 1, left((it + 1) & 1));
+        }
         table((u + 1) % NS, n + 1);
 #pragma unroll
         for (int s = 0; s < S; s++) {
@@ -535,7 +560,10 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
               hrow(A, B, r - 1);
               ehalf(B, Z, r - 1, s);
             }
-            if (RARE(smp)) sample(B, r - 1, st);
+            if (RARE(sampled(r - 1)) && (last || s < S - 1)) {
+              if (first) leave(B, it & 1);
+              else sample(r - 1, st, field(B));
+            }
           }
         }
         const int O = (u - S + 2 * NS) % NS;
@@ -555,12 +583,13 @@ __global__ __launch_bounds__(64 * (STREAM_T / S)) __attribute__((amdgpu_waves_pe
 {
   __shared__ D2 lv[stream_lds_v(MODE, PML, C, S)];
   __shared__ double li[stream_lds_i(MODE, C, S)];
+  __shared__ D2 ls[2 * 3 * C * 64];
   // workgroup b runs on XCD b % 8: each XCD takes a contiguous eighth of the strips
   const int per = (a.ns + 7) / 8;
   const int id = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
   if (id >= a.ns) return;
   const StreamStrip t = cload(a.strips + id);
-  strip_body<MODE, FLAV, PML, C, S, PF>(a, t, lv, li);
+  strip_body<MODE, FLAV, PML, C, S, PF>(a, t, lv, li, ls);
 }
 
 // Both kinds of strips in one launch (kind 0 interior, 1 frame): small grids, whose
@@ -571,12 +600,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   constexpr int C = stream_cols(MODE, FLAV), nv0 = stream_lds_v(MODE, 0, C, 2), nv1 = stream_lds_v(MODE, 1, 1, 2);
   __shared__ D2 lv[nv0 > nv1 ? nv0 : nv1];
   __shared__ double li[stream_lds_i(MODE, C, 2)];
+  __shared__ D2 ls[2 * 3 * C * 64];
   const int per = (a.ns + 7) / 8;
   const int id = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
   if (id >= a.ns) return;
   const StreamStrip t = cload(a.strips + id);
-  if (t.kind == 0) strip_body<MODE, FLAV, 0, stream_cols(MODE, FLAV), 2, STREAM_IPF>(a, t, lv, li);
-  else strip_body<MODE, FLAV, 1, 1, 2, stream_pf(MODE, FLAV)>(a, t, lv, li);
+  if (t.kind == 0) strip_body<MODE, FLAV, 0, stream_cols(MODE, FLAV), 2, STREAM_IPF>(a, t, lv, li, ls);
+  else strip_body<MODE, FLAV, 1, 1, 2, stream_pf(MODE, FLAV)>(a, t, lv, li, ls);
 }
 
 // The auxiliaries of the cells without UPML from the fields (the steps do not keep
@@ -784,12 +814,16 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
         t.r1 = std::min(r1, r + rows);
         t.b0 = r == 1 ? 0 : r - T;
         t.bl = std::min(X - 1, t.r1 - 1 + T);
+        t.s0 = t.r1;
         for (int q = 0; q < 4; q++) {
+          // the sides that pass through the strip and the rows they take
           const StreamSide &g = s->side[q];
-          const int a0 = g.horiz ? t.j0 : t.r0, a1 = g.horiz ? t.j1 : t.r1;
-          const int b0 = g.horiz ? t.r0 : t.j0, b1 = g.horiz ? t.r1 : t.j1;
-          const bool line = (g.fi >= a0 && g.fi < a1) || (g.fi - 1 >= a0 && g.fi - 1 < a1);
-          if (g.n > 0 && line && g.lo < b1 && g.lo + g.n > b0) t.smp = 1;
+          const int ra = std::max(t.r0, g.horiz ? g.lo : g.fi - 1), rb = std::min(t.r1, g.horiz ? g.lo + g.n : g.fi + 1);
+          const int ca = std::max(t.j0, g.horiz ? g.fi - 1 : g.lo), cb = std::min(t.j1, g.horiz ? g.fi + 1 : g.lo + g.n);
+          if (g.n <= 0 || ra >= rb || ca >= cb) continue;
+          t.smp |= 1 << q;
+          t.s0 = std::min(t.s0, ra);
+          t.s1 = std::max(t.s1, rb);
         }
         v.push_back(t);
       }
