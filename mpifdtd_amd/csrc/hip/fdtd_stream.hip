@@ -186,7 +186,17 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
 #pragma unroll
       for (int x = 0; x < 2; x++) cs[s][x] = a.c[0][w * S + s + 1][x] - (PML ? 0.0 : a.c[0][w * S + s][x]);
   }
+  // interior MPI: e^{i kx x} of the newest row, loaded an iteration ahead (loaded where a
+  // row meets a scatterer, it was a wait for two loads in turn: 1056 x 1056 with a
+  // cylinder 59.9 -> 52.2 us per 8 steps, 44 without the cylinder)
+  D2 exr = d2(0, 0), exn = d2(0, 0);
+  auto ahead = [&](int r) {
+    if (!WK) return;
+    exr = exn;
+    exn = cload2(a.ex + __builtin_amdgcn_readfirstlane(rowc(r)));
+  };
   auto wave = [&](int v, int r, int c, double ie) -> D2 {
+    if (WK) return mul(ie == 0.0 ? 0.0 : ie - 1.0, cmulp(exr, ey[c]));
     CAS(StreamArgs) R = rare_args();
     const double f = ie == 0.0 || !R->on[v] ? 0.0 : ie - 1.0;
     return mul(f, cmulp(cload2(R->ex + __builtin_amdgcn_readfirstlane(rowc(r))), ey[c]));
@@ -572,6 +582,7 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
       }
     }
     table(0, row0);
+    ahead(row0);
     for (int it0 = 0; it0 < nit; it0 += NS) {
 #pragma unroll
       for (int u = 0; u < NS; u++) {
@@ -579,6 +590,7 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
         // (left by return, not skipped: a join with the skipping path would again wait for every load)
         if (RARE(it >= nit)) return;
         const int n = row0 + it;
+        ahead(n + 1);
         if (first) settle(u, n);
         else flag(u, n);
         if (first) load((u + PF) % NS, n + PF);
