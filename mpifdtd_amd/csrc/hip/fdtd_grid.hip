@@ -1383,10 +1383,17 @@ struct fdtd_grid {
   int sCap, sFill;
   long sTb0;
   int ctrSet;            // FP32: the fused kernel samples the contour
-  // FP32: stream of the sample packing, binning and running DFT, beside the next
+  // stream of the sample packing, binning and running DFT, beside the next
   // block's step kernel; ev_k orders it after the block that took the samples
   hipStream_t ns;
   hipEvent_t ev_k;
+  // FP64 blocked grids: the group of samples being filled and its steps so far, the time
+  // of its first, and per group the event after its packing (wanted: packed on ns)
+  int smpGrp, smpN;
+  double smpTime;
+  double2 *smpBuf;
+  hipEvent_t smpFree[2];
+  int smpUsed[2];
   int overlap;  // -1: by grid size (on up to NTFF_OVERLAP_CELLS cells), 0: in order on the step stream, 1: on ns
   double *cosA, *sinA, *cosB, *sinB;
   double coef;
@@ -1792,6 +1799,25 @@ __global__ __launch_bounds__(256) void k_ctr_combine(const V *smp, Contour ct, l
 
 #define NTFF_OVERLAP_CELLS (8L << 20)
 
+// the stream of the work on samples that the null stream's last launch took, ordered after it
+static int ntff_stream(fdtd_grid *g, hipStream_t *st)
+{
+  // beside the next block on small grids, whose step kernel leaves the GPU
+  // partly idle; in order on large ones, whose step kernel fills it (there the
+  // overlap only stretches both)
+  const bool ovl = g->overlap < 0 ? g->ncell <= NTFF_OVERLAP_CELLS : g->overlap != 0;
+  *st = 0;
+  if (!ovl) return FDTD_OK;
+  if (!g->ns) {
+    HIPCHK(hipStreamCreateWithFlags(&g->ns, hipStreamNonBlocking));
+    HIPCHK(hipEventCreateWithFlags(&g->ev_k, hipEventDisableTiming));
+  }
+  HIPCHK(hipEventRecord(g->ev_k, 0));
+  HIPCHK(hipStreamWaitEvent(g->ns, g->ev_k, 0));
+  *st = g->ns;
+  return FDTD_OK;
+}
+
 // after a launch of n steps of an FP32 grid: pack the samples, bin every step at
 // its time and add them to the running DFT, on the grid's NTFF stream (the
 // next block's step kernel runs meanwhile)
@@ -1801,20 +1827,9 @@ static int grid_bin_samples(void *ctx, const float2 *samples, int n, const doubl
   if (n > g->nbuf) return fdtd_fail(FDTD_EINVAL, "%d steps exceed the %d-step sample buffers", n, g->nbuf);
   for (int s = 1; s < n; s++)
     if (times[s] != times[0] + s) return fdtd_fail(FDTD_ESTATE, "steps of a block are not consecutive");
-  // beside the next block on small grids, whose step kernel leaves the GPU
-  // partly idle; in order on large ones, whose step kernel fills it (there the
-  // overlap only stretches both)
-  const bool ovl = g->overlap < 0 ? g->ncell <= NTFF_OVERLAP_CELLS : g->overlap != 0;
-  hipStream_t st = 0;
-  if (ovl) {
-    if (!g->ns) {
-      HIPCHK(hipStreamCreateWithFlags(&g->ns, hipStreamNonBlocking));
-      HIPCHK(hipEventCreateWithFlags(&g->ev_k, hipEventDisableTiming));
-    }
-    HIPCHK(hipEventRecord(g->ev_k, 0));
-    HIPCHK(hipStreamWaitEvent(g->ns, g->ev_k, 0));
-    st = g->ns;
-  }
+  hipStream_t st;
+  int rc = ntff_stream(g, &st);
+  if (rc) return rc;
   const dim3 cgrid((g->ct.total + 255) / 256, n);
   if (g->ntn) {
     // binned step by step: [cell][nbuf], the first n steps of each cell; the DFT reads the same buffers
@@ -1917,7 +1932,7 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
   const int P = std::max(1, g->ct.total);
   // blocked paths bin a whole block of steps at once: sample buffers for as many
   const bool upml = d->flavour == FDTD_FLAVOUR_MPI || d->flavour == FDTD_FLAVOUR_PLAIN;
-  g->nbuf = d->precision == FDTD_FP32 ? FAST_MAX_T : (upml ? STREAM_T : 1);
+  g->nbuf = d->precision == FDTD_FP32 ? FAST_MAX_T : (upml ? STREAM_GROUP : 1);
   // the sample buffer: E samples of every cell, then H, nbuf steps per cell
   // (the binning's records address both from cE)
   HIPCHK(dev_malloc(&g->cE, (size_t)2 * g->nbuf * P * sizeof(double2)));
@@ -2026,6 +2041,8 @@ extern "C" int fdtd_hip_grid_destroy(fdtd_grid *g)
   if (g->ns) {
     (void)hipStreamDestroy(g->ns);
     (void)hipEventDestroy(g->ev_k);
+    for (int q = 0; q < 2; q++)
+      if (g->smpFree[q]) (void)hipEventDestroy(g->smpFree[q]);
     g->ns = nullptr;
   }
   for (int f = 0; f < 9 && !g->F64; f++) (void)dev_free(g->F[f]);
@@ -2239,29 +2256,66 @@ extern "C" int fdtd_hip_grid_get_eps(fdtd_grid *g, int which, double *host)
   return FDTD_OK;
 }
 
+// The samples of the group of steps taken since the last call: packed, binned and added
+// to the running DFT, on the NTFF stream beside the steps that follow.  Two launches'
+// steps together, so that the streams wait for each other (10 us) half as often: 531 x 402
+// TE with the per-step NTFF, 16 steps: 196 us in order, 178 beside.
+static int stream_samples(fdtd_grid *g)
+{
+  const int n = g->smpN, q = g->smpGrp;
+  if (!n) return FDTD_OK;
+  g->smpN = 0;
+  hipStream_t st;
+  int rc = ntff_stream(g, &st);
+  if (rc) return rc;
+  const dim3 cgrid((g->ct.total + 255) / 256, n);
+  double2 *E = g->cE, *H = g->cH;
+  long ss = 1, sp = g->nbuf;
+  if (!g->ntn) {
+    const size_t col = (size_t)dft_stage(g, n, g->smpTime, st) * g->ct.total;
+    E = g->sE + col;
+    H = g->sH + col;
+    ss = g->ct.total;
+    sp = 1;
+  }
+  hipLaunchKernelGGL(k_ctr_combine<double2>, cgrid, dim3(256), 0, st, g->smpBuf, g->ct, ss, sp, E, H);
+  if (st) {
+    if (!g->smpFree[q]) HIPCHK(hipEventCreateWithFlags(&g->smpFree[q], hipEventDisableTiming));
+    HIPCHK(hipEventRecord(g->smpFree[q], st));
+    g->smpUsed[q] = 1;
+  }
+  g->smpGrp = q ^ 1;
+  if (g->ntn) {
+    launch_bin(g, n, g->smpTime, st);
+    if (g->nf) dft_add(g, E, H, ss, sp, n, (long)llround(g->smpTime) - 1, st);
+  }
+  HIPCHK(hipGetLastError());
+  return FDTD_OK;
+}
+
 // n (<= STREAM_T) consecutive steps of an FP64 UPML grid in one launch, and the NTFF
 // work of all of them
 static int stream_block(fdtd_grid *g, const fdtd_step_params *p, int n)
 {
   const bool ctr = g->ct.total > 0 && (g->ntn || g->nf);
-  const double2 *smp = nullptr;
-  int rc = stream_steps(g->st, &g->F64, p, n, ctr ? 1 : 0, &smp);
+  const int q = g->smpGrp;
+  if (ctr && !g->smpN && g->smpUsed[q]) {
+    // this group's last samples are still being packed
+    HIPCHK(hipStreamWaitEvent(0, g->smpFree[q], 0));
+    g->smpUsed[q] = 0;
+  }
+  double2 *smp = nullptr;
+  int rc = stream_steps(g->st, &g->F64, p, n, ctr ? q * STREAM_GROUP + g->smpN : -1, &smp);
   if (rc) return rc;
   set_F64(g);
   g->auxok = 0;
   if (!ctr) return FDTD_OK;
-  const dim3 cgrid((g->ct.total + 255) / 256, n);
-  if (g->ntn) {
-    hipLaunchKernelGGL(k_ctr_combine<double2>, cgrid, dim3(256), 0, 0, smp, g->ct, 1L, (long)g->nbuf, g->cE, g->cH);
-    launch_bin(g, n, p[0].time, 0);
-    if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, n, (long)llround(p[0].time) - 1, 0);
-  } else {
-    const size_t col = (size_t)dft_stage(g, n, p[0].time, 0) * g->ct.total;
-    hipLaunchKernelGGL(k_ctr_combine<double2>, cgrid, dim3(256), 0, 0, smp, g->ct, (long)g->ct.total, 1L, g->sE + col,
-                       g->sH + col);
+  if (!g->smpN) {
+    g->smpTime = p[0].time;
+    g->smpBuf = smp;
   }
-  HIPCHK(hipGetLastError());
-  return FDTD_OK;
+  g->smpN += n;
+  return g->smpN + STREAM_T > STREAM_GROUP ? stream_samples(g) : FDTD_OK;
 }
 
 // n (<= split_depth) steps of a split-field or NS grid in one launch
@@ -2297,7 +2351,7 @@ extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int 
     if (rc) return rc;
     i += m;
   }
-  return FDTD_OK;
+  return stream_samples(g);
 }
 
 extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
@@ -2310,9 +2364,17 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
   }
   if (g->sp && !g->general && !g->nf && split_depth(g->sp)) return split_block(g, p, 1);
   if (g->st && !g->general) {
-    if (stream_follows(g->st, p)) return stream_block(g, p, 1);
-    int rc = go_general(g, false);
-    if (rc) return rc;
+    int rc;
+    if (stream_follows(g->st, p)) {
+      if ((rc = stream_block(g, p, 1))) return rc;
+      return stream_samples(g);
+    }
+    if ((rc = go_general(g, false))) return rc;
+  }
+  if (g->st) {
+    // the samples of earlier blocks first
+    int rc = stream_samples(g);
+    if (rc || (rc = ntff_sync(g))) return rc;
   }
   GridPtrs gp;
   for (int f = 0; f < 9; f++) gp.F[f] = g->F[f];
@@ -2468,6 +2530,7 @@ extern "C" int fdtd_hip_grid_reset(fdtd_grid *g)
   if (!g) return fdtd_fail(FDTD_EINVAL, "null argument");
   int rc0 = ntff_sync(g);
   if (rc0) return rc0;
+  g->smpN = 0;
   for (int f = 0; f < 9; f++)
     if (g->F[f]) HIPCHK(hipMemset(g->F[f], 0, g->ncell * sizeof(double2)));
   for (int a = 0; a < 3 && g->ntn; a++) HIPCHK(hipMemset(g->ntb[a], 0, g->ntn * sizeof(double2)));

@@ -56,6 +56,10 @@ struct FastStep {
 };
 
 #define STREAM_T 8  // steps per launch of the FP64 UPML path
+// contour samples of an FP64 blocked grid: two groups, one filled by the steps while
+// the binning reads the other, of two launches' steps each
+#define STREAM_GROUP (2 * STREAM_T)
+#define STREAM_SAMPLES (2 * STREAM_GROUP)
 #define FAST_MAX_T 16
 // rows of a UPML tile's block: the 4-wavefront UPML body (4 x 8 rows, the
 // merged, split and two-stream shapes, and batches) and the wide bodies of the
@@ -152,7 +156,7 @@ int stream_set_eps(StreamState *s, double *const *eps);
 void stream_reset(StreamState *s);
 long stream_steps_done(const StreamState *s);
 bool stream_follows(const StreamState *s, const fdtd_step_params *p);
-int stream_steps(StreamState *s, double2 **F, const fdtd_step_params *p, int n, int samples, const double2 **smp);
+int stream_steps(StreamState *s, double2 **F, const fdtd_step_params *p, int n, int at, double2 **smp);
 int stream_fill_aux(StreamState *s, double2 *F);
 
 // the same for the split-field and non-standard solvers (fdtd_stream_split.hip), whose

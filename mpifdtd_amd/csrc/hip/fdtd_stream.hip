@@ -1013,9 +1013,10 @@ static void launch(const StreamState *s, StreamArgs a)
 }
 
 // n <= STREAM_T steps from the arrays *F, which then hold the new state (the
-// buffer is swapped with the state's own); with samples, the contour's after
-// every step in *smp ([n][3][total])
-int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int samples, const D2 **smp)
+// buffer is swapped with the state's own); with at >= 0, the contour's samples
+// after every step in the entries [at, at + n) of the state's STREAM_SAMPLES, from
+// *smp on ([n][3][total])
+int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int at, D2 **smp)
 {
   if (n < 1 || n > STREAM_T) return fdtd_fail(FDTD_EINVAL, "bad number of steps %d", n);
   int rc;
@@ -1055,16 +1056,17 @@ int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int s
     a.ps[q + 1][0] = s->ps.x;
     a.ps[q + 1][1] = s->ps.y;
   }
-  if (samples) {
+  if (at >= 0) {
+    if (at + n > STREAM_SAMPLES) return fdtd_fail(FDTD_EINVAL, "bad sample entry %d", at);
+    const size_t e = 3 * (size_t)s->ctot;
     if (!s->csamp) {
-      const size_t b = (size_t)STREAM_T * 3 * s->ctot * sizeof(D2);
-      HIPCHK(dev_malloc(&s->csamp, b));
-      HIPCHK(hipMemset(s->csamp, 0, b));
+      HIPCHK(dev_malloc(&s->csamp, STREAM_SAMPLES * e * sizeof(D2)));
+      HIPCHK(hipMemset(s->csamp, 0, STREAM_SAMPLES * e * sizeof(D2)));
     }
-    a.csamp = s->csamp;
+    a.csamp = s->csamp + at * e;
     a.ctot = s->ctot;
     memcpy(a.side, s->side, sizeof a.side);
-    if (smp) *smp = s->csamp;
+    if (smp) *smp = a.csamp;
   }
   if (tm && mpi) launch<FDTD_MODE_TM, FDTD_FLAVOUR_MPI>(s, a);
   else if (tm) launch<FDTD_MODE_TM, FDTD_FLAVOUR_PLAIN>(s, a);
