@@ -279,9 +279,10 @@ int fdtd_hip_batch_create(fdtd_grid *const *grids, const fdtd_step_params *p0, c
 int fdtd_hip_batch_run(fdtd_hip_batch *b, int blocks);
 /* the interior tiles of a block are launched, then the UPML tiles
  * (FAST_LAUNCH_SPLIT; AUTO and MERGED mean the same here), or the two side by
- * side on two streams (FAST_LAUNCH_TWO_STREAMS); the *_PML8 shapes run the
- * UPML tiles as 8 wavefronts, the *_W8 shapes the interior tiles as well
- * (R >= 8).  Default: FAST_LAUNCH_TWO_STREAMS_PML8. */
+ * side on two streams (FAST_LAUNCH_TWO_STREAMS).  The *_PML8 and *_W8 shapes run
+ * wide UPML tiles (48 rows as 16 wavefronts), all of them but SPLIT_PML8 the
+ * interior tiles as 8 wavefronts (R >= 8), and the two on two streams the TE
+ * instances beside the TM ones.  Default: FAST_LAUNCH_TWO_STREAMS_PML8. */
 int fdtd_hip_batch_set_launch_mode(fdtd_hip_batch *b, int mode);
 int fdtd_hip_batch_sync(fdtd_hip_batch *b, int *steps_done);
 int fdtd_hip_batch_destroy(fdtd_hip_batch *b);

@@ -36,8 +36,8 @@ int fdtd_batch_run(fdtd_batch *b);
 int fdtd_batch_run_blocks(fdtd_batch *b, int blocks);
 int fdtd_batch_sync(fdtd_batch *b, int *steps_done);
 /* launch shape of every block (FAST_LAUNCH_* of fdtd_hip.h; TWO_STREAMS_PML8 by default).
- * FDTD_EINVAL for values outside the enum and for the *_P16 shapes, whose
- * 16-wavefront UPML tiles exist for single grids only. */
+ * FDTD_EINVAL for values outside the enum and for the *_P16 shapes, which exist
+ * for single grids only. */
 int fdtd_batch_set_launch_mode(fdtd_batch *b, int mode);
 int fdtd_batch_size(const fdtd_batch *b);
 /* instance i: NPXa, NPYa, off (1: padded MPI layout), arraySize */

@@ -74,9 +74,10 @@ class Batch:
         self.T, self.R = T, R
 
     def set_launch_mode(self, mode):
-        """2: interior tiles then UPML tiles; 3: the two side by side on two streams; 4 / 5: 2 / 3
-        with the UPML tiles as 8 wavefronts (5 is the default); 6 / 7: 4 / 5 with the interior
-        tiles as 8 wavefronts as well (FAST_LAUNCH_* of fdtd_hip.h)."""
+        """2: interior tiles then UPML tiles; 3: the two side by side on two streams; 4: 2 with wide
+        UPML tiles (48 rows as 16 wavefronts); 6: 4 with the interior tiles as 8 wavefronts; 5 (the
+        default) and 7: 6 with the TE instances beside the TM ones on two streams (FAST_LAUNCH_* of
+        fdtd_hip.h)."""
         check(N.lib().fdtd_batch_set_launch_mode(self._h, int(mode)), "fdtd_batch_set_launch_mode")
 
     def run(self):

@@ -890,13 +890,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(fast_interi
 // KQ: the queues pulled, 0 UPML tiles, 1 interior tiles, 2 both (UPML first).
 // A one-queue instantiation carries one tile body only, so it runs at that
 // body's register budget.
-// W8 (one-queue instantiations): the tiles as 8 wavefronts (512 threads), UPML
-// tiles of 32 rows as 8 x 4 rows, interior tiles of 4R rows as 8 x R/2 rows.
-template <int MODE, int R, int KQ, int W8 = 0>
-__global__ __launch_bounds__(W8 ? 512 : 256)
-__attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(W8 ? R / 2 : R) : 1))) void k_fast_batch(FastArgs a)
+// WIDE (one-queue instantiations): interior tiles of 4R rows as 8 wavefronts of R/2
+// rows (512 threads), UPML tiles of FAST_UPML_ROWS_WIDE = 48 rows as 16 wavefronts of
+// 3 rows (1024 threads): of a tile's rows 48 - 2T - 1 are core rows where a 32-row tile
+// keeps 32 - 2T - 1 (T = 8: 31 and 15); a block of 32 TM instances of 400 x 400 cells
+// took 285 us with 32-row tiles as 8 wavefronts of 4 rows, 238 with these.
+template <int MODE, int R, int KQ, int WIDE = 0>
+__global__ __launch_bounds__(!WIDE ? 256 : (KQ == 0 ? 1024 : 512))
+__attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(WIDE ? R / 2 : R) : (WIDE ? 4 : 1)))) void k_fast_batch(FastArgs a)
 {
-  static_assert(!W8 || (KQ != 2 && R >= 8), "8-wavefront bodies: one queue, R >= 8");
+  static_assert(!WIDE || (KQ != 2 && R >= 8), "wide bodies: one queue, R >= 8");
   __shared__ int s_tid;
   for (int k = (KQ == 1 ? 1 : 0); k < (KQ == 0 ? 1 : 2); k++) {
     // the queue in 8 contiguous parts, one per XCD (workgroup b runs on XCD b % 8):
@@ -917,8 +920,8 @@ __attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(W8 ? R / 2 : R)
         pp++;  // this part is empty (uniform: s_tid is shared)
         continue;
       }
-      if constexpr (W8) {
-        if (KQ == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, 4, 1, 1, 0, 8>(a, a.qoff[0] + tid);
+      if constexpr (WIDE) {
+        if (KQ == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, FAST_UPML_ROWS_WIDE / 16, 1, 1, 0, 16>(a, a.qoff[0] + tid);
         else fast_tile<MODE, FDTD_FLAVOUR_MPI, R / 2, 0, 1, 0, 8>(a, a.qoff[1] + tid);
       } else {
         if (KQ != 1 && k == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, 8, 1, 1, 0>(a, a.qoff[0] + tid);
@@ -1179,7 +1182,6 @@ struct FastState {
   // rows of the UPML tiles (FAST_UPML_ROWS or FAST_UPML_ROWS_WIDE, by launch
   // shape: each UPML body covers one height) and the height the lists hold
   int upmlRows = FAST_UPML_ROWS, tilesU = -1;
-  bool batch = false;  // an instance of a batch: its UPML bodies are the 32-row ones
   int cur = 0, pending = 0;
   int src_on = 0;
   double prev_c_re = 0, prev_c_im = 0;
@@ -1714,9 +1716,9 @@ int fast_state_flush(FastState *s)
   // the UPML bodies of the *_PML8, *_W8 and *_P16 shapes cover the wide tiles
   {
     const int lm = mode;
-    const bool wide = !s->batch && (lm == FAST_LAUNCH_SPLIT_PML8 || lm == FAST_LAUNCH_TWO_STREAMS_PML8 ||
-                                    lm == FAST_LAUNCH_SPLIT_W8 || lm == FAST_LAUNCH_TWO_STREAMS_W8 ||
-                                    lm == FAST_LAUNCH_SPLIT_P16 || lm == FAST_LAUNCH_TWO_STREAMS_P16);
+    const bool wide = lm == FAST_LAUNCH_SPLIT_PML8 || lm == FAST_LAUNCH_TWO_STREAMS_PML8 ||
+                      lm == FAST_LAUNCH_SPLIT_W8 || lm == FAST_LAUNCH_TWO_STREAMS_W8 ||
+                      lm == FAST_LAUNCH_SPLIT_P16 || lm == FAST_LAUNCH_TWO_STREAMS_P16;
     s->upmlRows = wide ? FAST_UPML_ROWS_WIDE : FAST_UPML_ROWS;
     // R = 18 and 20 (72- and 80-row interior tiles) exist only as 8 wavefronts of 9 and 10 rows
     const int set = s->lmode;  // AUTO, whose choice depends on the grid, does not take them
@@ -1985,6 +1987,8 @@ int fast_state_gather(FastState *s, const Contour &ct, int off, double2 *cE, dou
 // host value changes between blocks, so the loop of blocks is captured once as
 // a hipGraph and replayed.
 
+enum { BATCH_KINDS = 1, BATCH_MODES = 2 };  // FastBatch::two_streams
+
 struct FastBatch {
   int n = 0, T = 4, R = 16;
   std::vector<FastState *> st;
@@ -1999,12 +2003,19 @@ struct FastBatch {
   int off[2][2] = {{0, 0}, {0, 0}};
   int nblk[2][2] = {{0, 0}, {0, 0}};  // workgroups per mode and queue
   hipStream_t stream = nullptr;
-  // two_streams: the UPML launches of a block on s2 beside the interior launches
-  // (fork and join by events, captured into the graph as dependencies);
-  // pml8 / inner8: the UPML / interior tiles as 8 wavefronts (the *_PML8, *_W8 shapes)
-  // Default: TWO_STREAMS_PML8, the fastest on the 64-instance sweep (260.7 G cell
-  // updates/s against 243.5 for SPLIT; every shape gives the same bits)
-  int two_streams = 1, pml8 = 1, inner8 = 0;
+  // wide / inner8: the UPML tiles of 48 rows / the interior tiles as 8 wavefronts.
+  // two_streams, the launches on s2 (fork and join by events, captured into the graph as
+  // dependencies): BATCH_KINDS the UPML tiles beside the interior tiles, both of
+  // 4-wavefront bodies; BATCH_MODES the TE instances beside the TM ones, each kind after
+  // the other.  A 16-wavefront UPML workgroup takes a compute unit for itself, so beside
+  // interior tiles it only waits for both of a unit's to end; the two modes fill each
+  // other's last rounds.  Per block of 8 steps, SPLIT / KINDS / MODES with the wide UPML
+  // tiles and 8-wavefront interior tiles: 16 uneven TM and TE instances 762 / 838 / 762 us,
+  // 4 of them 344 / 340 / 308; 32 TM of 400 x 400 238 / 239 / 238; before (32-row UPML
+  // tiles, KINDS) 821, 344 and 288.  Interior tiles as 4 wavefronts beside: 905 us and 339.
+  // Default: TWO_STREAMS_PML8 (every shape gives the same bits).
+  int two_streams = BATCH_MODES, wide = 1, inner8 = 0;
+  int tilesU = -1;  // rows of the UPML tiles in dtiles
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipGraph_t graph = nullptr;
@@ -2013,11 +2024,11 @@ struct FastBatch {
 };
 
 template <int MODE, int KQ>
-static void batch_launch_q(const FastArgs &a, int R, int nblk, bool w8, hipStream_t st)
+static void batch_launch_q(const FastArgs &a, int R, int nblk, bool wide, hipStream_t st)
 {
-  if (w8 && KQ == 0) hipLaunchKernelGGL((k_fast_batch<MODE, 8, 0, 1>), dim3(nblk), dim3(512), 0, st, a);
-  else if (w8 && R == 8) hipLaunchKernelGGL((k_fast_batch<MODE, 8, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
-  else if (w8 && R == 16) hipLaunchKernelGGL((k_fast_batch<MODE, 16, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
+  if (wide && KQ == 0) hipLaunchKernelGGL((k_fast_batch<MODE, 8, 0, 1>), dim3(nblk), dim3(1024), 0, st, a);
+  else if (wide && R == 8) hipLaunchKernelGGL((k_fast_batch<MODE, 8, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
+  else if (wide && R == 16) hipLaunchKernelGGL((k_fast_batch<MODE, 16, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
   else if (R == 4) hipLaunchKernelGGL((k_fast_batch<MODE, 4, KQ>), dim3(nblk), dim3(256), 0, st, a);
   else if (R == 8) hipLaunchKernelGGL((k_fast_batch<MODE, 8, KQ>), dim3(nblk), dim3(256), 0, st, a);
   else hipLaunchKernelGGL((k_fast_batch<MODE, 16, KQ>), dim3(nblk), dim3(256), 0, st, a);
@@ -2028,7 +2039,7 @@ static void batch_launch_mode(const FastBatch *b, const FastArgs &a, const int n
                               hipStream_t st_pml)
 {
   if (nblk[1] > 0) batch_launch_q<MODE, 1>(a, b->R, nblk[1], b->inner8 != 0, st);
-  if (nblk[0] > 0) batch_launch_q<MODE, 0>(a, b->R, nblk[0], b->pml8 != 0, st_pml);
+  if (nblk[0] > 0) batch_launch_q<MODE, 0>(a, b->R, nblk[0], b->wide != 0, st_pml);
 }
 
 static FastArgs batch_args(const FastBatch *b, int m)
@@ -2052,19 +2063,22 @@ static FastArgs batch_args(const FastBatch *b, int m)
 // one block of T steps for every unfinished instance, then the progress update
 static int batch_level(FastBatch *b)
 {
-  hipStream_t sp = b->stream;
-  if (b->two_streams) {
+  const bool both = b->nblk[0][0] + b->nblk[0][1] > 0 && b->nblk[1][0] + b->nblk[1][1] > 0;
+  const bool fork = b->two_streams == BATCH_KINDS || (b->two_streams == BATCH_MODES && both);
+  if (fork) {
     HIPCHK(hipEventRecord(b->ev_fork, b->stream));
     HIPCHK(hipStreamWaitEvent(b->s2, b->ev_fork, 0));
-    sp = b->s2;
   }
   for (int m = 0; m < 2; m++) {
     if (b->nblk[m][0] + b->nblk[m][1] == 0) continue;
     const FastArgs a = batch_args(b, m);
-    if (m == FDTD_MODE_TM) batch_launch_mode<FDTD_MODE_TM>(b, a, b->nblk[m], b->stream, sp);
-    else batch_launch_mode<FDTD_MODE_TE>(b, a, b->nblk[m], b->stream, sp);
+    hipStream_t si = b->stream, sp = b->stream;
+    if (b->two_streams == BATCH_KINDS) sp = b->s2;
+    else if (fork && m == FDTD_MODE_TE) si = sp = b->s2;
+    if (m == FDTD_MODE_TM) batch_launch_mode<FDTD_MODE_TM>(b, a, b->nblk[m], si, sp);
+    else batch_launch_mode<FDTD_MODE_TE>(b, a, b->nblk[m], si, sp);
   }
-  if (b->two_streams) {
+  if (fork) {
     HIPCHK(hipEventRecord(b->ev_join, b->s2));
     HIPCHK(hipStreamWaitEvent(b->stream, b->ev_join, 0));
   }
@@ -2095,6 +2109,60 @@ void fast_batch_destroy(FastBatch *b)
   delete b;
 }
 
+static void batch_shape(FastBatch *b, int mode)
+{
+  b->wide = mode >= FAST_LAUNCH_SPLIT_PML8;
+  b->two_streams = mode == FAST_LAUNCH_TWO_STREAMS ? BATCH_KINDS
+                   : mode == FAST_LAUNCH_TWO_STREAMS_PML8 || mode == FAST_LAUNCH_TWO_STREAMS_W8 ? BATCH_MODES : 0;
+  b->inner8 = b->wide && mode != FAST_LAUNCH_SPLIT_PML8 && b->R >= 8;
+}
+
+// The tile queues of the launch shape: per mode, the UPML queue then the interior queue,
+// instances largest first (longest-processing-time order).
+static int batch_tiles(FastBatch *b)
+{
+  const int rows = b->wide ? FAST_UPML_ROWS_WIDE : FAST_UPML_ROWS;
+  if (b->tilesU == rows) return FDTD_OK;
+  int rc;
+  std::vector<int> order(b->n);
+  for (int i = 0; i < b->n; i++) order[i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+    return (long)b->st[x]->h.NPX * b->st[x]->h.NPY > (long)b->st[y]->h.NPX * b->st[y]->h.NPY;
+  });
+  for (FastState *s : b->st) {
+    // (an instance stepped by itself meanwhile has its own tiles)
+    if ((rc = fast_state_set_blocking(s, b->T, b->R))) return rc;
+    s->upmlRows = rows;
+    if (s->tilesT != s->T || s->tilesR != s->R || s->tilesU != s->upmlRows)
+      if ((rc = build_tiles(s))) return rc;
+  }
+  std::vector<FastTile> all;
+  for (int m = 0; m < 2; m++) {
+    for (int k = 0; k < 2; k++) {
+      b->off[m][k] = (int)all.size();
+      for (int i : order) {
+        FastState *s = b->st[i];
+        if (s->d.mode != m) continue;
+        for (FastTile t : (k == 0 ? s->htp : s->hti)) {
+          t.inst = i;
+          all.push_back(t);
+        }
+      }
+      b->nt[m][k] = (int)all.size() - b->off[m][k];
+    }
+    // resident workgroups: at most one per compute unit for the UPML bodies,
+    // two for the interior body at R = 16
+    b->nblk[m][0] = std::min(b->nt[m][0], 256);
+    b->nblk[m][1] = std::min(b->nt[m][1], 512);
+  }
+  if (b->dtiles) (void)dev_free(b->dtiles);
+  b->dtiles = nullptr;
+  HIPCHK(dev_malloc(&b->dtiles, std::max<size_t>(1, all.size()) * sizeof(FastTile)));
+  if (!all.empty()) HIPCHK(hipMemcpy(b->dtiles, all.data(), all.size() * sizeof(FastTile), hipMemcpyHostToDevice));
+  b->tilesU = rows;
+  return FDTD_OK;
+}
+
 int fast_batch_create(FastState *const *st, const fdtd_step_params *p0, const int *steps, int n, int T, int R,
                       FastBatch **out)
 {
@@ -2106,15 +2174,10 @@ int fast_batch_create(FastState *const *st, const fdtd_step_params *p0, const in
   b->n = n;
   b->T = T;
   b->R = R;
+  batch_shape(b, FAST_LAUNCH_TWO_STREAMS_PML8);
   int rc;
   std::vector<FastInst> hinst(n);
   std::vector<FastBatchInst> hb(n);
-  // instance order of the queues: largest first (longest-processing-time order)
-  std::vector<int> order(n);
-  for (int i = 0; i < n; i++) order[i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-    return (long)st[x]->h.NPX * st[x]->h.NPY > (long)st[y]->h.NPX * st[y]->h.NPY;
-  });
   for (int i = 0; i < n; i++) {
     FastState *s = st[i];
     if (s->d.flavour != FDTD_FLAVOUR_MPI) {
@@ -2130,14 +2193,6 @@ int fast_batch_create(FastState *const *st, const fdtd_step_params *p0, const in
       fast_batch_destroy(b);
       return rc;
     }
-    s->batch = true;
-    s->upmlRows = FAST_UPML_ROWS;
-    if (s->tilesT != s->T || s->tilesR != s->R || s->tilesU != s->upmlRows) {
-      if ((rc = build_tiles(s))) {
-        fast_batch_destroy(b);
-        return rc;
-      }
-    }
     b->st.push_back(s);
     b->omega.push_back(p0[i].omega);
     b->steps.push_back(steps[i]);
@@ -2148,26 +2203,6 @@ int fast_batch_create(FastState *const *st, const fdtd_step_params *p0, const in
     hb[i].Ti = 0;
     hb[i].cur = s->cur;
   }
-  // tiles: per mode, the UPML queue then the interior queue, instances largest first
-  std::vector<FastTile> all;
-  for (int m = 0; m < 2; m++) {
-    for (int k = 0; k < 2; k++) {
-      b->off[m][k] = (int)all.size();
-      for (int i : order) {
-        FastState *s = st[i];
-        if (s->d.mode != m) continue;
-        for (FastTile t : (k == 0 ? s->htp : s->hti)) {
-          t.inst = i;
-          all.push_back(t);
-        }
-      }
-      b->nt[m][k] = (int)all.size() - b->off[m][k];
-    }
-    // resident workgroups: at most one per compute unit for the UPML bodies,
-    // two for the interior body at R = 16
-    b->nblk[m][0] = std::min(b->nt[m][0], 256);
-    b->nblk[m][1] = std::min(b->nt[m][1], 512);
-  }
   HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
   HIPCHK(hipStreamCreateWithFlags(&b->s2, hipStreamNonBlocking));
   HIPCHK(hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
@@ -2175,11 +2210,13 @@ int fast_batch_create(FastState *const *st, const fdtd_step_params *p0, const in
   HIPCHK(dev_malloc(&b->dinst, n * sizeof(FastInst)));
   HIPCHK(dev_malloc(&b->dbinst, n * sizeof(FastBatchInst)));
   HIPCHK(dev_malloc(&b->dsteps, (size_t)n * FAST_MAX_T * sizeof(FastStep)));
-  HIPCHK(dev_malloc(&b->dtiles, std::max<size_t>(1, all.size()) * sizeof(FastTile)));
   HIPCHK(dev_malloc(&b->dqctr, 32 * sizeof(int)));
   HIPCHK(hipMemcpy(b->dinst, hinst.data(), n * sizeof(FastInst), hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(b->dbinst, hb.data(), n * sizeof(FastBatchInst), hipMemcpyHostToDevice));
-  if (!all.empty()) HIPCHK(hipMemcpy(b->dtiles, all.data(), all.size() * sizeof(FastTile), hipMemcpyHostToDevice));
+  if ((rc = batch_tiles(b))) {
+    fast_batch_destroy(b);
+    return rc;
+  }
   HIPCHK(hipDeviceSynchronize());
   // depths of the first block, queue counters cleared
   hipLaunchKernelGGL(k_batch_advance, dim3((std::max(n, 4) + 255) / 256), dim3(256), 0, b->stream, b->dbinst, n, T,
@@ -2215,15 +2252,12 @@ int fast_batch_run(FastBatch *b, int blocks, int use_graph)
   return FDTD_OK;
 }
 
-// launch shape (FAST_LAUNCH_*): the UPML launches beside the interior launches on a
-// second stream or after them, each tile kind as 4 or 8 wavefronts (interior tiles
-// as 8 wavefronts only for R >= 8); applies to blocks queued afterwards (the
-// captured graph is rebuilt)
+// launch shape (FAST_LAUNCH_*); applies to blocks queued afterwards (the captured graph
+// is rebuilt)
 int fast_batch_set_launch(FastBatch *b, int mode)
 {
   if (mode < FAST_LAUNCH_AUTO || mode > FAST_LAUNCH_TWO_STREAMS_P16) return fdtd_fail(FDTD_EINVAL, "bad launch mode %d", mode);
-  // the 16-wavefront UPML tiles exist for single grids only (the batch kernel's
-  // tile bodies are 4 or 8 wavefronts)
+  // (these shapes were refused before the wide tiles of the others became 16 wavefronts)
   if (mode == FAST_LAUNCH_SPLIT_P16 || mode == FAST_LAUNCH_TWO_STREAMS_P16)
     return fdtd_fail(FDTD_EINVAL, "launch mode %d (16-wavefront UPML tiles) is not available for batches", mode);
   HIPCHK(hipStreamSynchronize(b->stream));
@@ -2231,11 +2265,8 @@ int fast_batch_set_launch(FastBatch *b, int mode)
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->gexec = nullptr;
   b->graph = nullptr;
-  b->two_streams = mode == FAST_LAUNCH_TWO_STREAMS || mode == FAST_LAUNCH_TWO_STREAMS_PML8 ||
-                   mode == FAST_LAUNCH_TWO_STREAMS_W8;
-  b->pml8 = mode >= FAST_LAUNCH_SPLIT_PML8;
-  b->inner8 = (mode == FAST_LAUNCH_SPLIT_W8 || mode == FAST_LAUNCH_TWO_STREAMS_W8) && b->R >= 8;
-  return FDTD_OK;
+  batch_shape(b, mode);
+  return batch_tiles(b);
 }
 
 // blocks still needed by the slowest instance
