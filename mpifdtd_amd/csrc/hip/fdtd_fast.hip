@@ -1203,6 +1203,9 @@ struct FastState {
   fast_post_fn post = nullptr;
   void *post_ctx = nullptr;
   double times[FAST_MAX_T];
+  // steps in the buffer being filled whose samples were not handed on yet, their times
+  int cfill = 0;
+  double ctimes[FAST_MAX_T];
   // launch shape (FAST_LAUNCH_*); the second stream and its events exist once the
   // two-stream shape has been used
   int lmode = 0, lmode_last = 0;  // setting; shape of the last launch
@@ -1707,10 +1710,37 @@ static int auto_shape(const FastState *s)
   return tm || mpi ? FAST_LAUNCH_MERGED : FAST_LAUNCH_TWO_STREAMS_P16;
 }
 
+// The samples of the blocks launched since the last call to the consumer (NTFF).
+int fast_state_post(FastState *s)
+{
+  if (!s->cfill) return FDTD_OK;
+  const int n = s->cfill, sb = s->cbuf;
+  s->cfill = 0;
+  if (!s->post) return FDTD_OK;
+  s->cused[sb] = true;
+  s->cbuf ^= 1;
+  return s->post(s->post_ctx, s->csampb[sb], n, s->ctimes, s->cfree[sb]);
+}
+
+static int run_block(FastState *s);
+
 int fast_state_flush(FastState *s)
+{
+  int rc = run_block(s);
+  return rc ? rc : fast_state_post(s);
+}
+
+// The queued steps in one launch.  Their contour samples are handed on once the buffer
+// has no room for another block: the step kernels and the NTFF stream wait for each
+// other that much less often (T = 8, two blocks: 1056 x 1056 TE with the per-step NTFF
+// @@ -> @@ us per 8 steps).
+static int run_block(FastState *s)
 {
   if (s->pending == 0) return FDTD_OK;
   int rc;
+  if (s->cfill && (s->cfill + s->pending > FAST_MAX_T || s->times[0] != s->ctimes[s->cfill - 1] + 1) &&
+      (rc = fast_state_post(s)))
+    return rc;
   const int Tsave = s->T;
   const int mode = s->lmode == FAST_LAUNCH_AUTO ? auto_shape(s) : s->lmode;
   // the UPML bodies of the *_PML8, *_W8 and *_P16 shapes cover the wide tiles
@@ -1742,8 +1772,8 @@ int fast_state_flush(FastState *s)
   const int sb = s->cbuf;
   if (s->csamp) {
     // this block's sample buffer was last read by the consumer two blocks ago
-    if (s->cused[sb]) HIPCHK(hipStreamWaitEvent(0, s->cfree[sb], 0));
-    a.csamp = s->csampb[sb];
+    if (s->cused[sb] && !s->cfill) HIPCHK(hipStreamWaitEvent(0, s->cfree[sb], 0));
+    a.csamp = s->csampb[sb] + (size_t)s->cfill * 3 * s->hct.total;
     a.ct = s->hct;
   }
   ProfRec pr;
@@ -1830,9 +1860,9 @@ int fast_state_flush(FastState *s)
   s->pending = 0;
   s->T = Tsave;
   if (s->csamp && s->post) {
-    s->cused[sb] = true;
-    s->cbuf ^= 1;
-    return s->post(s->post_ctx, s->csampb[sb], n, s->times, s->cfree[sb]);
+    memcpy(s->ctimes + s->cfill, s->times, n * sizeof *s->times);
+    s->cfill += n;
+    if (s->cfill + s->T > FAST_MAX_T) return fast_state_post(s);
   }
   return FDTD_OK;
 }
@@ -1874,7 +1904,7 @@ int fast_state_step(FastState *s, const fdtd_step_params *p, int *launched)
   s->pending++;
   if (launched) *launched = 0;
   if (s->pending >= s->T) {
-    if ((rc = fast_state_flush(s))) return rc;
+    if ((rc = run_block(s))) return rc;
     if (launched) *launched = 1;
   }
   return FDTD_OK;
@@ -1934,6 +1964,7 @@ int fast_state_import(FastState *s, int slot, const double2 *src, int NPYa, int 
 int fast_state_reset(FastState *s)
 {
   s->pending = 0;
+  s->cfill = 0;
   const size_t n = (size_t)s->h.NPX * s->h.pitch * sizeof(float2);
   for (int b = 0; b < 2; b++) {
     HIPCHK(hipMemset(s->h.f0[b], 0, n));

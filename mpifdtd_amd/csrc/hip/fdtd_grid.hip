@@ -2378,6 +2378,13 @@ static int split_block(fdtd_grid *g, const fdtd_step_params *p, int n)
 extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n)
 {
   if (!g || !p || n < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
+  if (g->fs) {
+    for (int i = 0; i < n; i++) {
+      int launched = 0, rc = fast_state_step(g->fs, p + i, &launched);
+      if (rc) return rc;
+    }
+    return fast_state_post(g->fs);
+  }
   const int depth = g->sp && !g->general ? split_depth(g->sp) : 0;
   for (int i = 0; i < n;) {
     int rc, m = 1;
@@ -2408,8 +2415,8 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
   if (!g || !p) return fdtd_fail(FDTD_EINVAL, "null argument");
   const fdtd_grid_desc &d = g->d;
   if (g->fs) {
-    int launched = 0;
-    return fast_state_step(g->fs, p, &launched);
+    int launched = 0, rc = fast_state_step(g->fs, p, &launched);
+    return rc ? rc : fast_state_post(g->fs);
   }
   if (g->sp && !g->general && !g->nf && split_depth(g->sp)) return split_block(g, p, 1);
   if (g->st && !g->general) {

@@ -178,6 +178,7 @@ int fast_state_set_coefs(FastState *s, const fdtd_coef_tables *t);
 int fast_state_set_inv_eps(FastState *s, double *const *eps_dev, int NPYa, int off);
 int fast_state_step(FastState *s, const fdtd_step_params *p, int *launched);
 int fast_state_flush(FastState *s);
+int fast_state_post(FastState *s);
 int fast_state_export(FastState *s, int slot, double2 *dst_dev, int NPYa, int off);
 int fast_state_import(FastState *s, int slot, const double2 *src_dev, int NPYa, int off);
 int fast_state_reset(FastState *s);

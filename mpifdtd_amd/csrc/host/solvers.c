@@ -648,7 +648,7 @@ static int kind_of(fdtd_method update);
 int solver_run(fdtd_method update, int n)
 {
   const int kind = kind_of(update);
-  if (kind < 0 || !slv_[kind].g || slv_[kind].blocked || finite_every_ > 0) return 0;
+  if (kind < 0 || !slv_[kind].g || finite_every_ > 0) return 0;
   fdtd_step_params p[RUN_STEPS];
   if (n > RUN_STEPS) n = RUN_STEPS;
   for (int i = 0; i < n; i++) {
