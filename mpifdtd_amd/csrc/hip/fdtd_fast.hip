@@ -2168,9 +2168,10 @@ static int batch_tiles(FastBatch *b)
       if ((rc = build_tiles(s))) return rc;
   }
   std::vector<FastTile> all;
-  for (int m = 0; m < 2; m++) {
+  int off[2][2], nt[2][2];
+  for (int m = 0; m < 2; m++)
     for (int k = 0; k < 2; k++) {
-      b->off[m][k] = (int)all.size();
+      off[m][k] = (int)all.size();
       for (int i : order) {
         FastState *s = b->st[i];
         if (s->d.mode != m) continue;
@@ -2179,17 +2180,29 @@ static int batch_tiles(FastBatch *b)
           all.push_back(t);
         }
       }
-      b->nt[m][k] = (int)all.size() - b->off[m][k];
+      nt[m][k] = (int)all.size() - off[m][k];
+    }
+  FastTile *tiles = nullptr;
+  HIPCHK(dev_malloc(&tiles, std::max<size_t>(1, all.size()) * sizeof(FastTile)));
+  if (!all.empty()) {
+    const hipError_t e = hipMemcpy(tiles, all.data(), all.size() * sizeof(FastTile), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)dev_free(tiles);
+      return fdtd_fail(FDTD_EHIP, "tiles of a batch: %s", hipGetErrorString(e));
+    }
+  }
+  if (b->dtiles) (void)dev_free(b->dtiles);
+  b->dtiles = tiles;
+  for (int m = 0; m < 2; m++) {
+    for (int k = 0; k < 2; k++) {
+      b->off[m][k] = off[m][k];
+      b->nt[m][k] = nt[m][k];
     }
     // resident workgroups: at most one per compute unit for the UPML bodies,
     // two for the interior body at R = 16
-    b->nblk[m][0] = std::min(b->nt[m][0], 256);
-    b->nblk[m][1] = std::min(b->nt[m][1], 512);
+    b->nblk[m][0] = std::min(nt[m][0], 256);
+    b->nblk[m][1] = std::min(nt[m][1], 512);
   }
-  if (b->dtiles) (void)dev_free(b->dtiles);
-  b->dtiles = nullptr;
-  HIPCHK(dev_malloc(&b->dtiles, std::max<size_t>(1, all.size()) * sizeof(FastTile)));
-  if (!all.empty()) HIPCHK(hipMemcpy(b->dtiles, all.data(), all.size() * sizeof(FastTile), hipMemcpyHostToDevice));
   b->tilesU = rows;
   return FDTD_OK;
 }
@@ -2296,8 +2309,15 @@ int fast_batch_set_launch(FastBatch *b, int mode)
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->gexec = nullptr;
   b->graph = nullptr;
+  const int old[3] = {b->wide, b->two_streams, b->inner8};
   batch_shape(b, mode);
-  return batch_tiles(b);
+  const int rc = batch_tiles(b);
+  if (rc) {  // the bodies must match the tiles: keep both as they were
+    b->wide = old[0];
+    b->two_streams = old[1];
+    b->inner8 = old[2];
+  }
+  return rc;
 }
 
 // blocks still needed by the slowest instance

@@ -1,4 +1,4 @@
-// fdtd_grid.hip -- FP64 reference-order UPML path for gfx950.
+// fdtd_grid.hip -- grids and their FP64 kernels of a step per launch for gfx950.
 //
 // One fdtd_grid is one simulation instance of one of the reference's four UPML
 // solvers (MPI TM/TE single rank, plain TM/TE).  Per reference update():
