@@ -1205,6 +1205,7 @@ struct FastState {
   double times[FAST_MAX_T];
   // steps in the buffer being filled whose samples were not handed on yet, their times
   int cfill = 0;
+  bool binned = false;  // the samples go to the per-step NTFF's binning, not to the running DFT alone
   double ctimes[FAST_MAX_T];
   // launch shape (FAST_LAUNCH_*); the second stream and its events exist once the
   // two-stream shape has been used
@@ -1699,13 +1700,17 @@ static int update_wave(FastState *s, const fdtd_step_params &p)
 // R = 16, us; merged / SPLIT_P16 / TWO_STREAMS_P16 on 500 x 400, 1056 x 1056 and
 // 2000 x 1500 cells): MPI TM 24/36/44, 34/43/54, 59/62/74; MPI TE 25/39/45, 53/48/57,
 // 100/72/83; plain TM 34/47/43, 51/50/58, 76/69/79; plain TE 60/66/46, 91/65/72,
-// 148/86/95.  The former two-launch shape of large grids (SPLIT, 4-wavefront tiles) took
-// 71, 93, 88 and 137 on 2000 x 1500.
+// 148/86/95.  The former two-launch shape of large grids
+// (SPLIT, 4-wavefront tiles) took 71, 93, 88 and 137 on 2000 x 1500.  The binning of the
+// per-step NTFF beside the launches moves plain TM's line up (76/89 on 1056 x 1056, 91/104
+// on 1300 x 1200, 127/123 on 1600 x 1400; merged / SPLIT_P16), the running DFT alone, which
+// needs little of the chip, MPI TM's down (47/47 on 800 x 800, 57/52, 67/61, 72/68).
 static int auto_shape(const FastState *s)
 {
   const size_t cells = (size_t)s->h.NPX * s->h.NPY;
   const bool tm = s->d.mode == FDTD_MODE_TM, mpi = s->d.flavour == FDTD_FLAVOUR_MPI;
-  const size_t line = tm ? (mpi ? (size_t)4 << 20 : (size_t)1 << 20) : (size_t)3 << 18;
+  const bool dft = s->csamp && !s->binned, bin = s->csamp && s->binned;
+  const size_t line = !tm ? (size_t)3 << 18 : mpi ? (size_t)(dft ? 1 : 4) << 20 : (size_t)(bin ? 2 : 1) << 20;
   if (cells >= line) return FAST_LAUNCH_SPLIT_P16;
   return tm || mpi ? FAST_LAUNCH_MERGED : FAST_LAUNCH_TWO_STREAMS_P16;
 }
@@ -1730,10 +1735,22 @@ int fast_state_flush(FastState *s)
   return rc ? rc : fast_state_post(s);
 }
 
-// The queued steps in one launch.  Their contour samples are handed on once the buffer
-// has no room for another block: the step kernels and the NTFF stream wait for each
-// other that much less often (T = 8, two blocks: 1056 x 1056 TE with the per-step NTFF
-// 98 -> 92 us per 8 steps).
+// Whether the contour samples are handed on once their buffer has no room for another
+// block, rather than after each: the step kernels and the NTFF stream wait for each other
+// less often.  With the per-step NTFF, T = 8, two blocks against one (us per 8 steps):
+// SPLIT_P16, 200 x 200 to 1600 x 1400 cells, MPI TE 50 / 54 to 132 / 146; merged, MPI TM
+// 37 / 41 on 200 x 200, 118 / 127 on 1600 x 1400.  Between these the merged launch leaves
+// room for one block's binning beside it and not for two's: MPI TM 60 / 54 on 800 x 800,
+// 77 / 73 on 1056 x 1056, 94 / 89 on 1300 x 1200; MPI TE, 44 / 42 on 500 x 400, is past it
+// at 800 x 800 (70 / 78).
+static bool group_samples(const FastState *s, int mode)
+{
+  const size_t cells = (size_t)s->h.NPX * s->h.NPY;
+  if (mode != FAST_LAUNCH_MERGED) return true;
+  return cells < (size_t)1 << 17 || cells >= (s->d.mode == FDTD_MODE_TM ? (size_t)2 << 20 : (size_t)1 << 19);
+}
+
+// The queued steps in one launch.
 static int run_block(FastState *s)
 {
   if (s->pending == 0) return FDTD_OK;
@@ -1862,7 +1879,7 @@ static int run_block(FastState *s)
   if (s->csamp && s->post) {
     memcpy(s->ctimes + s->cfill, s->times, n * sizeof *s->times);
     s->cfill += n;
-    if (s->cfill + s->T > FAST_MAX_T) return fast_state_post(s);
+    if (s->cfill + s->T > FAST_MAX_T || !group_samples(s, mode)) return fast_state_post(s);
   }
   return FDTD_OK;
 }
@@ -2360,7 +2377,7 @@ int fast_batch_sync(FastBatch *b, int *steps_done)
 // Contour of the per-step NTFF in the physical layout: the sides of `ct`
 // (solver-layout indices, `off` = 1 for the padded MPI layout) converted for
 // the fused kernel, and a sample buffer for FAST_MAX_T steps.
-int fast_state_set_contour(FastState *s, const Contour &ct, int off, fast_post_fn post, void *ctx)
+int fast_state_set_contour(FastState *s, const Contour &ct, int off, int binned, fast_post_fn post, void *ctx)
 {
   int rc;
   if ((rc = fast_state_flush(s))) return rc;
@@ -2405,6 +2422,7 @@ int fast_state_set_contour(FastState *s, const Contour &ct, int off, fast_post_f
     for (int b = 0; b < 2; b++) HIPCHK(dev_malloc(&s->csampb[b], (size_t)FAST_MAX_T * 3 * ct.total * sizeof(float2)));
     s->csamp = s->csampb[0];
   }
+  s->binned = binned != 0;
   s->post = post;
   s->post_ctx = ctx;
   return FDTD_OK;

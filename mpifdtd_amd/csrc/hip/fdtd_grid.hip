@@ -2029,7 +2029,7 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
     // the per-step time-domain NTFF: the fused kernel samples the contour after
     // every inner step, and each block's samples are binned step by step
     if (d->ntff_time && g->ct.total > 0) {
-      if ((rc = fast_state_set_contour(g->fs, g->ct, g->off, grid_bin_samples, g))) return rc;
+      if ((rc = fast_state_set_contour(g->fs, g->ct, g->off, 1, grid_bin_samples, g))) return rc;
       g->ctrSet = 1;
     }
   }
@@ -2814,7 +2814,7 @@ extern "C" int fdtd_hip_grid_set_dft(fdtd_grid *g, const double *omega, int nf)
   g->nf = nf;
   // the FP32 fused kernel samples the contour after every inner step
   if (g->fs && !g->ctrSet) {
-    if ((rc = fast_state_set_contour(g->fs, g->ct, g->off, grid_bin_samples, g))) return rc;
+    if ((rc = fast_state_set_contour(g->fs, g->ct, g->off, g->ntn ? 1 : 0, grid_bin_samples, g))) return rc;
     g->ctrSet = 1;
   }
   return FDTD_OK;

@@ -196,7 +196,8 @@ int fast_state_pitch(const FastState *s, int *pitch);
 // on its own stream after the block, and records `consumed` there once it has
 // read `samples` (the buffer is written again two blocks later)
 typedef int (*fast_post_fn)(void *ctx, const float2 *samples, int n, const double *times, hipEvent_t consumed);
-int fast_state_set_contour(FastState *s, const Contour &ct, int off, fast_post_fn post, void *ctx);
+// binned: the samples go to the per-step NTFF's binning (not to the running DFT alone)
+int fast_state_set_contour(FastState *s, const Contour &ct, int off, int binned, fast_post_fn post, void *ctx);
 int fast_state_set_blocking(FastState *s, int T, int R);
 int fast_state_set_launch_mode(FastState *s, int mode);
 int fast_state_get_launch_mode(const FastState *s);

@@ -47,7 +47,7 @@ class Simulator:
 
     def __init__(self, solver, model, fi, params=None, c0=0.7071, ntff_inset=5, point_source=False,
                  ntff_time=True, file_output=False, precision="fp64", T=None, R=16):
-        """precision "fp64": reference-order FP64 kernels; "fp32": fused FP32 kernels
+        """precision "fp64": FP64 kernels; "fp32": fused FP32 kernels
         advancing T steps per launch (with ntff_time on they sample the NTFF
         contour after every inner step)."""
         L = N.lib()
