@@ -19,7 +19,7 @@ the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of exactly this launch
 configuration under profiles/, divided by the block's event-timed duration in
 this run; the algorithmic rate (what an unblocked step would have to move) is
 reported beside it as "effective".  The DFT and far-field spectra of the FP32
-run are compared with the FP64 reference-order path on the same grid after
+run are compared with the FP64 path on the same grid after
 `--check-steps` steps.  The CPU baseline is the reference's own plain TM UPML
 step, compiled from its sources (oracle/_ref/ref_harness), timed on one host
 core and on all host cores before the GPU is touched.
@@ -479,7 +479,7 @@ def run_sweep81(args, m, cpu):
 # ---------------------------------------------------------------- other workloads
 
 def run_solvers_fp64(args, m):
-    """Every solver of enum SOLVER in its FP64 reference-order path on the mie1056
+    """Every solver of enum SOLVER in FP64 on the mie1056
     grid (the reference's cylinder; CW source for the MPI, split-field and NS
     solvers, Gaussian pulse for the plain UPML ones), without the per-step NTFF:
     the step rate of each over `steps` simulator_calc() calls after 20 untimed
@@ -511,7 +511,7 @@ def run_solvers_fp64(args, m):
         finally:
             sim.finish()
         per[name] = {"mcups": round(cells * steps / dt / 1e6, 1), "us_per_step": round(dt * 1e6 / steps, 2)}
-    return {"metric": "Mcell-updates/s, FP64 reference-order path, per solver", "value": per["NS_TE_2D"]["mcups"],
+    return {"metric": "Mcell-updates/s, FP64 path, per solver", "value": per["NS_TE_2D"]["mcups"],
             "unit": "Mcell-updates/s", "n_gpus": 1, "steps": steps, "warmup": 20,
             "ms_per_step": round(per["NS_TE_2D"]["us_per_step"] / 1e3, 5), "higher_is_better": True,
             "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "synthetic",
@@ -547,7 +547,7 @@ def run_sweep(args, m):
     ff = [b.far_field(i) for i in (0, 1)]
     check = {}
     if not args.no_check:
-        # two instances again through the FP64 reference-order single-instance path
+        # two instances again through the FP64 single-instance path
         for i in (0, 1):
             s = spec[i]
             solver = m.MPI_TM_UPML_2D if s["mode"] == "tm" else m.MPI_TE_UPML_2D
@@ -641,7 +641,7 @@ def run_single(args, m, cpu_ref):
     spec_steps = 8000 if wl == "mie1056" else 20000
     extra["spectra_per_s"] = round(1.0 / (spec_steps * ms_step * 1e-3 + t_ff), 4)
     if not args.no_check and args.precision == "fp32":
-        log("fp64 reference-order run for the far-field check")
+        log("fp64 run for the far-field check")
         ref = make_sim(m, "fp64", args.mode, total, workload=wl, ntff=args.ntff)
         t2 = time.perf_counter()
         ref.calc(total)
