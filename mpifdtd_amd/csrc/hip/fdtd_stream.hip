@@ -887,7 +887,8 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   // all run at once, both kinds in one launch (two workgroups of these registers fit a
   // compute unit).  8-step launches of the TM grids: 276 x 276 {8, 12} 31.9 us,
   // {16, 24} 39.1; 1056 x 1056 {16, 32} 58.5 us (one generation), {16, 24} 79.2 (two),
-  // {24, 48} 71.1, apart 38.0 + 45.4.  Larger grids run the two kinds apart.
+  // {24, 48} 71.1, apart 38.0 + 45.4 (since then 29.9 and 52.2 with the
+  // chosen pairs).  Larger grids run the two kinds apart.
   static const int rows[][2] = {{8, 12}, {8, 16}, {16, 24}, {16, 32}, {24, 48}, {32, 64}, {64, 128}};
   for (size_t q = 0; q < sizeof rows / sizeof rows[0]; q++) {
     const int Lf = rows[q][0], Li = rows[q][1];
