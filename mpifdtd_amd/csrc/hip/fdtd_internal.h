@@ -144,8 +144,9 @@ struct FastArgs {
 // ---------------------------------------------------------------- FP64 blocked path
 // (fdtd_stream.hip) of the UPML solvers; the grid owns the current arrays F, the
 // state the other buffers.  stream_follows: whether a step continues the steps
-// taken so far; a grid whose fields, structure or wave were changed in between
-// goes on step by step with the kernels that keep every auxiliary.
+// taken so far; a grid whose fields, structure or wave were changed in between, or
+// whose permittivity is outside the range the blocks take, goes on step by step with
+// the kernels that keep every auxiliary.
 struct StreamState;
 // bytes between the nine arrays of an FP64 state of n cells, which lie in one block
 static inline size_t stream_stride(size_t n) { return (n * sizeof(double2) + 255) & ~(size_t)255; }

@@ -99,6 +99,11 @@ __host__ __device__ constexpr int stream_ni(int mode) { return mode == FDTD_MODE
 __host__ __device__ constexpr int stream_cols(int mode, int flav) { return mode == FDTD_MODE_TE && flav == FDTD_FLAVOUR_PLAIN ? 1 : 2; }
 __host__ __device__ constexpr int stream_pf(int mode, int flav) { return mode == FDTD_MODE_TM && flav == FDTD_FLAVOUR_MPI ? 2 : 1; }
 #define STREAM_IPF 2
+// Smallest 1/eps of the blocked steps: where 1/eps is smaller (or zero: a perfect
+// conductor), E is the source alone to all but its last bits, and J = D = eps (E - s)
+// cannot be formed from it; grids with such a cell step by the kernels that keep J and D.
+// At 2^-20 the difference keeps 32 bits.
+#define STREAM_IE_MIN 0x1p-20
 // LDS of the rows handed on: K - 1 pairs of wavefronts, two rows each
 __host__ __device__ constexpr int stream_lds_v(int mode, int pml, int C, int S) { return (STREAM_T / S - 1) * 2 * stream_nv(mode, pml) * C * 64; }
 __host__ __device__ constexpr int stream_lds_i(int mode, int C, int S) { return (STREAM_T / S - 1) * 2 * stream_ni(mode) * C * 64; }
@@ -703,13 +708,17 @@ __global__ __launch_bounds__(256) void k_stream_aux(StreamArgs a)
   }
 }
 
-// 1/eps, 0 on the ring of cells that are never updated
-__global__ __launch_bounds__(256) void k_stream_ie(const double *eps, int NPXa, int NPYa, double *ie)
+// 1/eps, 0 on the ring of cells that are never updated.  *odd is set if a cell's 1/eps
+// lies outside [STREAM_IE_MIN, 1 / STREAM_IE_MIN], NaN included.
+__global__ __launch_bounds__(256) void k_stream_ie(const double *eps, int NPXa, int NPYa, double *ie, int *odd)
 {
   const int j = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
   if (i >= NPXa || j >= NPYa) return;
   const size_t k = (size_t)i * NPYa + j;
-  ie[k] = (i == 0 || j == 0 || i == NPXa - 1 || j == NPYa - 1) ? 0.0 : 1.0 / eps[k];
+  const bool ring = i == 0 || j == 0 || i == NPXa - 1 || j == NPYa - 1;
+  const double v = 1.0 / eps[k];
+  ie[k] = ring ? 0.0 : v;
+  if (!ring && !(fabs(v) >= STREAM_IE_MIN && fabs(v) <= 1.0 / STREAM_IE_MIN)) *odd = 1;
 }
 
 // ---------------------------------------------------------------- host
@@ -726,6 +735,8 @@ struct StreamState {
   double *ie[2];
   double *xt, *yt;
   D2 *exy;
+  int *odd;    // device flag of k_stream_ie, per map
+  bool isodd;  // a permittivity the blocked steps do not take
   StreamStrip *strips;  // interior, then frame
   int nint, nfrm;
   int xlo, xhi;
@@ -766,6 +777,7 @@ int stream_create(const fdtd_grid_desc &d, int off, const Contour &ct, StreamSta
   HIPCHK(dev_malloc(&s->xt, (size_t)s->NPXa * 8 * sizeof(double)));
   HIPCHK(dev_malloc(&s->yt, (size_t)s->NPYa * 6 * sizeof(double)));
   HIPCHK(dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)));
+  HIPCHK(dev_malloc(&s->odd, 2 * sizeof(int)));
   s->ctot = ct.total;
   for (int q = 0; q < 4; q++) {
     const Seg &g = ct.s[q];
@@ -792,6 +804,7 @@ void stream_destroy(StreamState *s)
   (void)dev_free(s->xt);
   (void)dev_free(s->yt);
   (void)dev_free(s->exy);
+  (void)dev_free(s->odd);
   (void)dev_free(s->strips);
   (void)dev_free(s->csamp);
   delete s;
@@ -923,9 +936,13 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
 int stream_set_eps(StreamState *s, double *const *eps)
 {
   const dim3 blk(64, 4), grd((s->NPYa + 63) / 64, (s->NPXa + 3) / 4);
+  int odd[2] = {0, 0};
+  HIPCHK(hipMemset(s->odd, 0, sizeof odd));
   for (int e = 0; e < 2; e++)
-    if (s->ie[e]) hipLaunchKernelGGL(k_stream_ie, grd, blk, 0, 0, eps[e], s->NPXa, s->NPYa, s->ie[e]);
+    if (s->ie[e]) hipLaunchKernelGGL(k_stream_ie, grd, blk, 0, 0, eps[e], s->NPXa, s->NPYa, s->ie[e], s->odd + e);
   HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpy(odd, s->odd, sizeof odd, hipMemcpyDeviceToHost));
+  s->isodd = odd[0] || odd[1];
   return FDTD_OK;
 }
 
@@ -935,7 +952,7 @@ long stream_steps_done(const StreamState *s) { return s->steps; }
 // whether a step with these parameters continues the steps taken so far
 bool stream_follows(const StreamState *s, const fdtd_step_params *p)
 {
-  if (!s->coefs) return false;
+  if (!s->coefs || s->isodd) return false;
   if (!s->steps) return true;
   return p->angle_deg == s->angle && p->k == s->k && p->omega == s->omega && p->time == s->time + 1 &&
          (s->d.flavour == FDTD_FLAVOUR_MPI || s->d.mode == FDTD_MODE_TM ||
