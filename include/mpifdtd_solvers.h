@@ -29,6 +29,7 @@
 #ifndef MPIFDTD_SOLVERS_H
 #define MPIFDTD_SOLVERS_H
 
+#include <stddef.h>
 #include "mpifdtd_field.h"
 
 #ifdef __cplusplus
@@ -159,6 +160,10 @@ double *fdtdTE_upml_getEps(void);
  * holds no UPML cell: there getState reads zero and setState drops the values */
 int fdtd_solver_getState(int which, double *out);
 int fdtd_solver_setState(int which, const double *in);
+/* the field a getter of `solver` (enum SOLVER) returns, which 0..2 (TM Ez Hx Hy, TE Ex Ey
+ * Hz), into `out` of `cells` = NPXa*NPYa complex doubles, whether that solver is the active
+ * one or not; FDTD_ESTATE if it is not initialised, FDTD_EINVAL if its size is another */
+int fdtd_solver_readField(int solver, int which, double *out, size_t cells);
 /* time-domain NTFF accumulators (which 0..2: Ux Uy Wz / Wx Wy Uz), 360*arraySize complex */
 int fdtd_solver_getNTFFTime(int which, double *out);
 /* frequency-domain far field of the current fields, 360 complex (re,im):

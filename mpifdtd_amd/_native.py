@@ -140,6 +140,7 @@ def lib():
     # solver extensions
     sig("fdtd_solver_getState", I, I, dp)
     sig("fdtd_solver_setState", I, I, dp)
+    sig("fdtd_solver_readField", I, I, I, dp, ctypes.c_size_t)
     sig("fdtd_solver_getNTFFTime", I, I, dp)
     sig("fdtd_solver_farField", I, dp)
     sig("fdtd_solver_farFieldNoAlloc", I, dp)

@@ -620,6 +620,15 @@ int fdtd_solver_getState(int which, double *out)
   if (active_ < 0) return FDTD_ESTATE;
   return fdtd_hip_grid_get_field(slv_[active_].g, which, out);
 }
+int fdtd_solver_readField(int solver, int which, double *out, size_t cells)
+{
+  static const int kinds[] = {SLV_SPLIT_TM, SLV_SPLIT_TE, SLV_TM, SLV_TE, SLV_MPI_TM, SLV_MPI_TE, SLV_NS_TM, SLV_NS_TE};
+  if (!out || which < 0 || which > 2 || solver < TM_2D || solver > NS_TE_2D) return FDTD_EINVAL;
+  const solver_t *s = &slv_[kinds[solver]];
+  if (!s->g) return FDTD_ESTATE;
+  if (cells != (size_t)s->NPXa * s->NPYa) return FDTD_EINVAL;
+  return fdtd_hip_grid_get_field(s->g, slot_of_[which], out);
+}
 int fdtd_solver_setState(int which, const double *in)
 {
   if (active_ < 0) return FDTD_ESTATE;
