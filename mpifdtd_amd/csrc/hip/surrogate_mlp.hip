@@ -628,10 +628,18 @@ extern "C" int mlp_destroy(mlp_net *net)
 static int fwd_ld(const mlp_net *n) { return n->maxW + 8; }
 static bool fwd_fits(const mlp_net *n) { return 2u * 16 * fwd_ld(n) * sizeof(bf16_t) <= 65536; }
 
+// Whether k_mlp_forward's workgroups, which read and write 16 rows each in any order, may
+// run on these buffers: y apart from x, or row for row in its place.
+static bool fwd_apart(const float *x, size_t nx, const float *y, size_t ny)
+{
+  const uintptr_t a = (uintptr_t)x, b = (uintptr_t)y;
+  return b >= a + nx * sizeof(float) || a >= b + ny * sizeof(float) || (a == b && nx == ny);
+}
+
 extern "C" int mlp_forward(mlp_net *n, const float *x, int B, float *y)
 {
   if (!n || !x || !y || B < 1 || B > n->Bmax) return fdtd_fail(FDTD_EINVAL, "mlp_forward: bad argument");
-  if (fwd_fits(n)) {
+  if (fwd_fits(n) && fwd_apart(x, (size_t)B * n->l[0].K, y, (size_t)B * n->l[n->L - 1].N)) {
     FwdArgs a = {};
     a.n = n->L;
     a.B = B;
