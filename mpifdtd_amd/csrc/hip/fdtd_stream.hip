@@ -167,7 +167,11 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
 #pragma unroll
   for (int c = 0; c < C; c++) ey[c] = a.ey[min(col + c, NPY - 1)];
   const bool lin = col < NPY;             // frame: lanes past the grid hold zeros
-  const int lc = min(col, NPY - C);       // clamped column of the loads
+  // Clamped column of the loads: lanes past the core's halo, which a narrow frame strip has
+  // many of, take its last column, or rows whose scatterer only they see would form its
+  // wave (80 x 80 with a cylinder in the middle, us per 8 steps: plain TE 76 -> 39, MPI TM
+  // 42 -> 29).
+  const int lc = min(col, min(NPY - C, t.j1 + STREAM_T - 1));
   double y0 = 1, y1 = 1, y2 = 1, y3 = 1, s2p = 2, s2m = 2;
   bool ypml = false;
   if (PML) {

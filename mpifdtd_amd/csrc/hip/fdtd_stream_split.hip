@@ -90,7 +90,8 @@ __global__ __launch_bounds__(64 * SP_K) __attribute__((amdgpu_waves_per_eu(2))) 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int NPX = a.NPXa, NPY = a.NPYa;
-  const int col = t.bj + lane, lc = min(col, NPY - 1);
+  const int col = t.bj + lane;
+  const int lc = min(col, min(NPY - 1, t.j1 + sp_t(PH)));  // lanes past the halo take its last column
   const bool lin = col < NPY;  // lanes past the grid hold zeros
   D2 V[NSL][NV];
   double I[NSL][NI];
