@@ -8,9 +8,10 @@
 //                                                       (fdtdTM_upml.c:54-66, fdtdTE_upml.c:168-192)
 // The arithmetic of every update here keeps the reference's operation order and
 // is compiled without FMA contraction, so results agree with the CPU solver to
-// rounding of the device sin/cos/exp only.  The UPML solvers' steps run in blocks
-// (fdtd_stream.hip), which agree to rounding; these kernels take over where a
-// grid's state, structure or wave is changed between steps.
+// rounding of the device sin/cos/exp only.  Longer runs of steps go in blocks
+// (fdtd_stream.hip, fdtd_stream_split.hip), which agree to rounding; these kernels take
+// the few steps that cost less one by one, and grids whose state, structure or wave
+// is changed between steps.
 //
 // HBM layout: each complex field is an array of double2 (re, im), row-major
 // k = i*NPYa + j (j = y contiguous), exactly the reference's layout, so host
@@ -674,8 +675,8 @@ __global__ __launch_bounds__(256) void k_te_h(GridPtrs g, Tabs t)
 // ---------------------------------------------------------------- NTFF (time domain)
 
 // gather the contour samples of this step: E value (signed) and the averaged,
-// signed H value of every contour cell, sp elements per cell
-__global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Contour ct, int sp, double2 *cE, double2 *cH)
+// signed H value of every contour cell.  F: the first of the grid's nine arrays, `stride` bytes apart
+__global__ __launch_bounds__(256) void k_ntff_gather(const double2 *F, size_t stride, Contour ct, double2 *cE, double2 *cH)
 {
   const int p = blockIdx.x * 256 + threadIdx.x;
   if (p >= ct.total) return;
@@ -684,15 +685,17 @@ __global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Co
   const Seg &sg = ct.s[s];
   const int c = p - sg.off;
   const long k = sg.k0 + (long)c * sg.dk;
-  const double2 e = F[sg.ef][k];
-  const double2 h0 = F[sg.hf][k], h1 = F[sg.hf][k + sg.hnb];
+  const double2 *E = (const double2 *)((const char *)F + sg.ef * stride);
+  const double2 *H = (const double2 *)((const char *)F + sg.hf * stride);
+  const double2 e = E[k];
+  const double2 h0 = H[k], h1 = H[k + sg.hnb];
   double2 ev, hv;
   ev.x = sg.es * e.x;
   ev.y = sg.es * e.y;
   hv.x = sg.hs * (h0.x + h1.x);
   hv.y = sg.hs * (h0.y + h1.y);
-  cE[(size_t)p * sp] = ev;
-  cH[(size_t)p * sp] = hv;
+  cE[p] = ev;
+  cH[p] = hv;
 }
 
 #define NT_GUARD_DEV 4  // guard bins allocated before and after the accumulators
@@ -700,6 +703,8 @@ __global__ __launch_bounds__(256) void k_ntff_gather(const double2 *const *F, Co
 #define NTFF_GRP 32    // sample groups per workgroup of k_ntff_bin
 #define NTFF_RUN 16    // samples per group and part
 #define NTFF_AHEAD 4   // records of a group's run loaded together
+#define NTFF_STEPS 16  // steps of the sample buffer that the records address (nbuf)
+static_assert(NTFF_STEPS == FAST_MAX_T && NTFF_STEPS == STREAM_GROUP, "a launch's steps fill the sample buffer");
 
 // Binning of n consecutive steps per launch.
 //
@@ -735,7 +740,9 @@ struct BinPart {
   int row, arr;   // angle, target array
 };
 
-template <int NS>
+// ONE: the samples of one step, packed ([cell], E then H): [cell][nbuf] leaves each in a
+// cache line of its own.
+template <int NS, bool ONE = false>
 __global__ __launch_bounds__(NTFF_GRP * NS) void k_ntff_bin(const double2 *cS, int n,
                                                              const BinPart *parts, const BinRec *rec, double2 *U0,
                                                              double2 *U1, double2 *U2, int arraySize, long tb0,
@@ -758,7 +765,7 @@ __global__ __launch_bounds__(NTFF_GRP * NS) void k_ntff_bin(const double2 *cS, i
   auto value = [&](int p) {
     // p: the element of the sample's first step; padding (p < 0) and lanes past
     // n read nothing
-    return (p >= 0 && act) ? cS[p + s] : make_double2(0.0, 0.0);
+    return (p >= 0 && act) ? cS[ONE ? (unsigned)p / NTFF_STEPS : p + s] : make_double2(0.0, 0.0);
   };
   // the run is taken NTFF_AHEAD records at a time: all their record loads, then
   // all their value loads, are in flight together (a record's value load
@@ -1395,7 +1402,6 @@ struct fdtd_grid {
   size_t ncell;
   double2 *F[9];
   double2 *F64;  // FP64 grids: the block that holds F[]
-  double2 **Fdev;  // device copy of F[] for the gather kernel
   double *eps[3];
   double *tab;
   Tabs tabs;
@@ -1428,6 +1434,8 @@ struct fdtd_grid {
   // block's step kernel; ev_k orders it after the block that took the samples
   hipStream_t ns;
   hipEvent_t ev_k;
+  hipEvent_t ev_n;  // orders the null stream after ns, where it has work since it was last waited for (nsBusy)
+  int nsBusy;
   // FP64 blocked grids: the group of samples being filled and its steps so far, the time
   // of its first, and per group the event after its packing (wanted: packed on ns)
   int smpGrp, smpN;
@@ -1755,24 +1763,34 @@ static int build_bin_groups(fdtd_grid *g)
   return FDTD_OK;
 }
 
-// the first n steps of the samples in cE / cH ([cell][nbuf]) into the accumulators
+// where the samples of n steps are packed for the binning: step s of cell c at E[s + c * sp]
+static long bin_samples(const fdtd_grid *g, int n, double2 **E, double2 **H)
+{
+  *E = g->cE;
+  *H = n == 1 ? g->cE + g->ct.total : g->cH;
+  return n == 1 ? 1 : g->nbuf;
+}
+
+// the n steps of samples that bin_samples placed into the accumulators
 static void launch_bin(fdtd_grid *g, int n, double time0, hipStream_t st)
 {
   const fdtd_grid_desc &d = g->d;
   const long tb0 = (long)llround(time0) - 1;
   const int useCoef = d.flavour == FDTD_FLAVOUR_PLAIN ? 0 : 1;
   if (g->nparts <= 0) return;
-#define NTFF_BIN(NS)                                                                                              \
-  hipLaunchKernelGGL(k_ntff_bin<NS>, dim3(g->nparts), dim3(NTFF_GRP * NS), 0, st, g->cE, n, g->binPart, g->binRec,        \
+#define NTFF_BIN(NS, ONE)                                                                                            \
+  hipLaunchKernelGGL((k_ntff_bin<NS, ONE>), dim3(g->nparts), dim3(NTFF_GRP * NS), 0, st, g->cE, n, g->binPart, g->binRec, \
                      g->nt[0], g->nt[1], g->nt[2], d.array_size, tb0, g->coef, useCoef)
-  if (n <= 2)
-    NTFF_BIN(2);
+  if (n == 1)
+    NTFF_BIN(2, true);
+  else if (n == 2)
+    NTFF_BIN(2, false);
   else if (n <= 4)
-    NTFF_BIN(4);
+    NTFF_BIN(4, false);
   else if (n <= 8)
-    NTFF_BIN(8);
+    NTFF_BIN(8, false);
   else
-    NTFF_BIN(16);
+    NTFF_BIN(16, false);
 #undef NTFF_BIN
 }
 
@@ -1859,10 +1877,12 @@ static int ntff_stream(fdtd_grid *g, hipStream_t *st)
   if (!g->ns) {
     HIPCHK(hipStreamCreateWithFlags(&g->ns, hipStreamNonBlocking));
     HIPCHK(hipEventCreateWithFlags(&g->ev_k, hipEventDisableTiming));
+    HIPCHK(hipEventCreateWithFlags(&g->ev_n, hipEventDisableTiming));
   }
   HIPCHK(hipEventRecord(g->ev_k, 0));
   HIPCHK(hipStreamWaitEvent(g->ns, g->ev_k, 0));
   *st = g->ns;
+  g->nsBusy = 1;
   return FDTD_OK;
 }
 
@@ -1880,11 +1900,13 @@ static int grid_bin_samples(void *ctx, const float2 *samples, int n, const doubl
   if (rc) return rc;
   const dim3 cgrid((g->ct.total + 255) / 256, n);
   if (g->ntn) {
-    // binned step by step: [cell][nbuf], the first n steps of each cell; the DFT reads the same buffers
-    hipLaunchKernelGGL(k_ctr_combine<float2>, cgrid, dim3(256), 0, st, samples, g->ct, 1L, (long)g->nbuf, g->cE, g->cH);
+    // binned step by step; the DFT reads the same buffers
+    double2 *E, *H;
+    const long sp = bin_samples(g, n, &E, &H);
+    hipLaunchKernelGGL(k_ctr_combine<float2>, cgrid, dim3(256), 0, st, samples, g->ct, 1L, sp, E, H);
     HIPCHK(hipEventRecord(consumed, st));
     launch_bin(g, n, times[0], st);
-    if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, n, (long)llround(times[0]) - 1, st);
+    if (g->nf) dft_add(g, E, H, 1, sp, n, (long)llround(times[0]) - 1, st);
   } else if (g->nf) {
     // DFT only: staged, the DFT runs over up to sCap steps at once
     const size_t col = (size_t)dft_stage(g, n, times[0], st) * g->ct.total;
@@ -1903,6 +1925,17 @@ static int grid_bin_samples(void *ctx, const float2 *samples, int n, const doubl
 static int ntff_sync(fdtd_grid *g)
 {
   if (g->ns) HIPCHK(hipStreamSynchronize(g->ns));
+  g->nsBusy = 0;
+  return FDTD_OK;
+}
+
+// the null stream after the work on samples that was put on ns
+static int ntff_join(fdtd_grid *g)
+{
+  if (!g->nsBusy) return FDTD_OK;
+  HIPCHK(hipEventRecord(g->ev_n, g->ns));
+  HIPCHK(hipStreamWaitEvent(0, g->ev_n, 0));
+  g->nsBusy = 0;
   return FDTD_OK;
 }
 
@@ -1947,8 +1980,6 @@ extern "C" int fdtd_hip_grid_create(const fdtd_grid_desc *d, fdtd_grid **out)
     HIPCHK(hipMemset(g->F64, 0, 9 * stride));
     set_F64(g);
   }
-  HIPCHK(dev_malloc(&g->Fdev, 9 * sizeof(double2 *)));
-  HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
   for (int e = 0; e < 3; e++) {
     HIPCHK(dev_malloc(&g->eps[e], g->ncell * sizeof(double)));
     HIPCHK(hipMemset(g->eps[e], 0, g->ncell * sizeof(double)));
@@ -2089,13 +2120,13 @@ extern "C" int fdtd_hip_grid_destroy(fdtd_grid *g)
   if (g->ns) {
     (void)hipStreamDestroy(g->ns);
     (void)hipEventDestroy(g->ev_k);
+    (void)hipEventDestroy(g->ev_n);
     for (int q = 0; q < 2; q++)
       if (g->smpFree[q]) (void)hipEventDestroy(g->smpFree[q]);
     g->ns = nullptr;
   }
   for (int f = 0; f < 9 && !g->F64; f++) (void)dev_free(g->F[f]);
   (void)dev_free(g->F64);
-  (void)dev_free(g->Fdev);
   for (int e = 0; e < 3; e++) (void)dev_free(g->eps[e]);
   (void)dev_free(g->nsc);
   (void)dev_free(g->tab);
@@ -2142,15 +2173,11 @@ static int ensure_aux(fdtd_grid *g)
 static int go_general(fdtd_grid *g, bool steps_only)
 {
   // the split solvers' blocks form the sums from the split components, which a caller may set apart
-  if (g->sp && !steps_only && !g->general) {
-    g->general = 1;
-    HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
-  }
+  if (g->sp && !steps_only) g->general = 1;
   if (!g->st || g->general || (steps_only && !stream_steps_done(g->st))) return FDTD_OK;
   int rc = ensure_aux(g);
   if (rc) return rc;
   g->general = 1;
-  HIPCHK(hipMemcpy(g->Fdev, g->F, 9 * sizeof(double2 *), hipMemcpyHostToDevice));
   return FDTD_OK;
 }
 
@@ -2318,8 +2345,8 @@ static int stream_samples(fdtd_grid *g)
   int rc = ntff_stream(g, &st);
   if (rc) return rc;
   const dim3 cgrid((g->ct.total + 255) / 256, n);
-  double2 *E = g->cE, *H = g->cH;
-  long ss = 1, sp = g->nbuf;
+  double2 *E, *H;
+  long ss = 1, sp = bin_samples(g, n, &E, &H);
   if (!g->ntn) {
     const size_t col = (size_t)dft_stage(g, n, g->smpTime, st) * g->ct.total;
     E = g->sE + col;
@@ -2375,62 +2402,14 @@ static int split_block(fdtd_grid *g, const fdtd_step_params *p, int n)
   return rc;
 }
 
-extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n)
+// One step by the kernels of a step, which keep every array.
+static int one_step(fdtd_grid *g, const fdtd_step_params *p)
 {
-  if (!g || !p || n < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
-  if (g->fs) {
-    for (int i = 0; i < n; i++) {
-      int launched = 0, rc = fast_state_step(g->fs, p + i, &launched);
-      if (rc) return rc;
-    }
-    return fast_state_post(g->fs);
-  }
-  const int depth = g->sp && !g->general ? split_depth(g->sp) : 0;
-  for (int i = 0; i < n;) {
-    int rc, m = 1;
-    if (depth && !g->nf) {
-      while (m < depth && i + m < n && p[i + m].angle_deg == p[i].angle_deg && p[i + m].k == p[i].k) m++;
-      rc = split_block(g, p + i, m);
-    } else if (g->st && !g->general && stream_follows(g->st, p + i)) {
-      const fdtd_step_params &a = p[i];
-      while (m < STREAM_T && i + m < n) {
-        const fdtd_step_params &b = p[i + m];
-        if (b.time != a.time + m || b.angle_deg != a.angle_deg || b.k != a.k || b.omega != a.omega || b.dot_x != a.dot_x ||
-            b.dot_y != a.dot_y || b.use_x != a.use_x || b.use_y != a.use_y)
-          break;
-        m++;
-      }
-      rc = stream_block(g, p + i, m);
-    } else {
-      rc = fdtd_hip_grid_step(g, p + i);
-    }
-    if (rc) return rc;
-    i += m;
-  }
-  return stream_samples(g);
-}
-
-extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
-{
-  if (!g || !p) return fdtd_fail(FDTD_EINVAL, "null argument");
   const fdtd_grid_desc &d = g->d;
-  if (g->fs) {
-    int launched = 0, rc = fast_state_step(g->fs, p, &launched);
-    return rc ? rc : fast_state_post(g->fs);
-  }
-  if (g->sp && !g->general && !g->nf && split_depth(g->sp)) return split_block(g, p, 1);
-  if (g->st && !g->general) {
-    int rc;
-    if (stream_follows(g->st, p)) {
-      if ((rc = stream_block(g, p, 1))) return rc;
-      return stream_samples(g);
-    }
-    if ((rc = go_general(g, false))) return rc;
-  }
   if (g->st) {
-    // the samples of earlier blocks first
-    int rc = stream_samples(g);
-    if (rc || (rc = ntff_sync(g))) return rc;
+    // the samples of earlier blocks first, and the auxiliaries the blocks do not keep
+    int rc;
+    if ((rc = stream_samples(g)) || (rc = ntff_join(g)) || (rc = ensure_aux(g))) return rc;
   }
   GridPtrs gp;
   for (int f = 0; f < 9; f++) gp.F[f] = g->F[f];
@@ -2521,20 +2500,62 @@ extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p)
     }
   }
   HIPCHK(hipGetLastError());
+  const size_t stride = stream_stride(g->ncell);
   if (g->ntn && g->ct.total > 0) {
-    hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, (const double2 *const *)g->Fdev,
-                       g->ct, g->nbuf, g->cE, g->cH);
+    double2 *E, *H;
+    const long sp = bin_samples(g, 1, &E, &H);
+    hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, g->F64, stride, g->ct, E, H);
     launch_bin(g, 1, p->time, 0);
-    if (g->nf) dft_add(g, g->cE, g->cH, 1, g->nbuf, 1, (long)llround(p->time) - 1, 0);
+    if (g->nf) dft_add(g, E, H, 1, sp, 1, (long)llround(p->time) - 1, 0);
     HIPCHK(hipGetLastError());
   } else if (g->nf && g->ct.total > 0) {
     const size_t col = (size_t)dft_stage(g, 1, p->time, 0) * g->ct.total;
-    hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, (const double2 *const *)g->Fdev,
-                       g->ct, 1, g->sE + col, g->sH + col);
+    hipLaunchKernelGGL(k_ntff_gather, dim3((g->ct.total + 255) / 256), dim3(256), 0, 0, g->F64, stride, g->ct, g->sE + col,
+                       g->sH + col);
     HIPCHK(hipGetLastError());
   }
-  return FDTD_OK;
+  return g->st && !g->general ? stream_note(g->st, p) : FDTD_OK;
 }
+
+extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n)
+{
+  if (!g || !p || n < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
+  if (g->fs) {
+    for (int i = 0; i < n; i++) {
+      int launched = 0, rc = fast_state_step(g->fs, p + i, &launched);
+      if (rc) return rc;
+    }
+    return fast_state_post(g->fs);
+  }
+  for (int i = 0; i < n;) {
+    // m steps from i that a block can hold, `few` of them at most by the kernels of a step
+    int rc, m = 1, few = 1;
+    const fdtd_step_params &a = p[i];
+    if (g->sp && !g->general && !g->nf && split_depth(g->sp)) {  // (blocks take no contour samples)
+      few = split_few(g->sp);
+      while (m < split_depth(g->sp) && i + m < n && p[i + m].angle_deg == a.angle_deg && p[i + m].k == a.k) m++;
+      rc = m > few ? split_block(g, p + i, m) : FDTD_OK;
+    } else if (g->st && !g->general && stream_follows(g->st, &a)) {
+      few = stream_few(g->st, g->ntn ? g->ct.total : 0);
+      while (m < STREAM_T && i + m < n) {
+        const fdtd_step_params &b = p[i + m];
+        if (b.time != a.time + m || b.angle_deg != a.angle_deg || b.k != a.k || b.omega != a.omega || b.dot_x != a.dot_x ||
+            b.dot_y != a.dot_y || b.use_x != a.use_x || b.use_y != a.use_y)
+          break;
+        m++;
+      }
+      rc = m > few ? stream_block(g, p + i, m) : FDTD_OK;
+    } else {
+      rc = g->st && !g->general ? go_general(g, false) : FDTD_OK;
+    }
+    for (int q = 0; q < m && m <= few && !rc; q++) rc = one_step(g, p + i + q);
+    if (rc) return rc;
+    i += m;
+  }
+  return stream_samples(g);
+}
+
+extern "C" int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p) { return fdtd_hip_grid_steps(g, p, 1); }
 
 // an FP32 grid's FP64 export buffer for slot f, zeroed when first made (the
 // ghost ring and the cells the export does not write stay zero)
@@ -2768,8 +2789,6 @@ extern "C" int fdtd_hip_grid_set_dft(fdtd_grid *g, const double *omega, int nf)
   if (!g || (nf > 0 && !omega) || nf < 0) return fdtd_fail(FDTD_EINVAL, "bad argument");
   if (nf > 0 && g->ct.total <= 0) return fdtd_fail(FDTD_ESTATE, "the grid has no NTFF contour");
   int rc;
-  // the split solvers' blocks take no contour samples
-  if (nf > 0 && g->sp && (rc = go_general(g, false))) return rc;
   if (g->fs && (rc = fast_state_flush(g->fs))) return rc;
   HIPCHK(hipDeviceSynchronize());
   (void)dev_free(g->dftOmega);

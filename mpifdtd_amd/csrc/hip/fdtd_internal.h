@@ -157,6 +157,10 @@ int stream_set_eps(StreamState *s, double *const *eps);
 void stream_reset(StreamState *s);
 long stream_steps_done(const StreamState *s);
 bool stream_follows(const StreamState *s, const fdtd_step_params *p);
+// stream_few: the most steps that take no more time one by one, on a grid whose per-step
+// NTFF samples `binned` contour cells; stream_note: such a step was taken
+int stream_few(const StreamState *s, int binned);
+int stream_note(StreamState *s, const fdtd_step_params *p);
 int stream_steps(StreamState *s, double2 **F, const fdtd_step_params *p, int n, int at, double2 **smp);
 int stream_fill_aux(StreamState *s, double2 *F);
 
@@ -170,6 +174,7 @@ int split_set_coefs(SplitState *s, const fdtd_coef_tables *t);
 int split_set_eps(SplitState *s, double *const *eps, const double *sx, const double *sy);
 int split_set_ns(SplitState *s, const double *nsc, double r2);
 int split_depth(const SplitState *s);
+int split_few(const SplitState *s);
 int split_steps(SplitState *s, double2 **F, const fdtd_step_params *p, int n);
 
 struct FastState;

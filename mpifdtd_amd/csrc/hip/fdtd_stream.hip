@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -712,17 +713,30 @@ __global__ __launch_bounds__(256) void k_stream_aux(StreamArgs a)
   }
 }
 
-// 1/eps, 0 on the ring of cells that are never updated.  *odd is set if a cell's 1/eps
-// lies outside [STREAM_IE_MIN, 1 / STREAM_IE_MIN], NaN included.
-__global__ __launch_bounds__(256) void k_stream_ie(const double *eps, int NPXa, int NPYa, double *ie, int *odd)
+// What the host asks of a permittivity map: whether a cell's 1/eps lies outside
+// [STREAM_IE_MIN, 1 / STREAM_IE_MIN], NaN included, and the box of the scatterer's cells.
+struct StreamMap {
+  int odd, i0, i1, j0, j1;  // rows [i0, i1], columns [j0, j1]
+};
+
+// 1/eps, 0 on the ring of cells that are never updated
+__global__ __launch_bounds__(256) void k_stream_ie(const double *eps, int NPXa, int NPYa, double *ie, StreamMap *m)
 {
   const int j = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
-  if (i >= NPXa || j >= NPYa) return;
+  const bool in = i < NPXa && j < NPYa, ring = i == 0 || j == 0 || i >= NPXa - 1 || j >= NPYa - 1;
   const size_t k = (size_t)i * NPYa + j;
-  const bool ring = i == 0 || j == 0 || i == NPXa - 1 || j == NPYa - 1;
-  const double v = 1.0 / eps[k];
-  ie[k] = ring ? 0.0 : v;
-  if (!ring && !(fabs(v) >= STREAM_IE_MIN && fabs(v) <= 1.0 / STREAM_IE_MIN)) *odd = 1;
+  const double v = in ? 1.0 / eps[k] : 1.0;
+  if (in) ie[k] = ring ? 0.0 : v;
+  if (!ring && !(fabs(v) >= STREAM_IE_MIN && fabs(v) <= 1.0 / STREAM_IE_MIN)) m->odd = 1;
+  // a wavefront holds 64 columns of one row; few of them still widen the box
+  const unsigned long long b = __ballot(!ring && v != 1.0);
+  if (!b || threadIdx.x) return;
+  const int j0 = j + __builtin_ctzll(b), j1 = j + 63 - __builtin_clzll(b);
+  auto now = [](int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  if (i < now(&m->i0)) atomicMin(&m->i0, i);
+  if (i > now(&m->i1)) atomicMax(&m->i1, i);
+  if (j0 < now(&m->j0)) atomicMin(&m->j0, j0);
+  if (j1 > now(&m->j1)) atomicMax(&m->j1, j1);
 }
 
 // ---------------------------------------------------------------- host
@@ -739,11 +753,11 @@ struct StreamState {
   double *ie[2];
   double *xt, *yt;
   D2 *exy;
-  int *odd;    // device flag of k_stream_ie, per map
-  bool isodd;  // a permittivity the blocked steps do not take
+  StreamMap *map;  // device, per 1/eps map
+  StreamMap seen;  // of all maps together
   StreamStrip *strips;  // interior, then frame
   int nint, nfrm;
-  int xlo, xhi;
+  int xlo, xhi, ylo, yhi;  // the box without UPML
   StreamSide side[4];
   int ctot;
   D2 *csamp;
@@ -781,7 +795,7 @@ int stream_create(const fdtd_grid_desc &d, int off, const Contour &ct, StreamSta
   HIPCHK(dev_malloc(&s->xt, (size_t)s->NPXa * 8 * sizeof(double)));
   HIPCHK(dev_malloc(&s->yt, (size_t)s->NPYa * 6 * sizeof(double)));
   HIPCHK(dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)));
-  HIPCHK(dev_malloc(&s->odd, 2 * sizeof(int)));
+  HIPCHK(dev_malloc(&s->map, 2 * sizeof(StreamMap)));
   s->ctot = ct.total;
   for (int q = 0; q < 4; q++) {
     const Seg &g = ct.s[q];
@@ -808,7 +822,7 @@ void stream_destroy(StreamState *s)
   (void)dev_free(s->xt);
   (void)dev_free(s->yt);
   (void)dev_free(s->exy);
-  (void)dev_free(s->odd);
+  (void)dev_free(s->map);
   (void)dev_free(s->strips);
   (void)dev_free(s->csamp);
   delete s;
@@ -864,6 +878,8 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   box(py, ylo, yhi);
   s->xlo = xlo;
   s->xhi = xhi;
+  s->ylo = ylo;
+  s->yhi = yhi;
   // the cells that keep auxiliaries: every updated one outside the box's rows or columns
   for (int i = 0; i < X; i++) xt[(size_t)i * 8 + 7] = i > 0 && i < X - 1 && (i < xlo || i >= xhi) ? 1.0 : 0.0;
   for (int j = 0; j < Y; j++) yt[5 * (size_t)Y + j] = j > 0 && j < Y - 1 && (j < ylo || j >= yhi) ? 1.0 : 0.0;
@@ -940,13 +956,15 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
 int stream_set_eps(StreamState *s, double *const *eps)
 {
   const dim3 blk(64, 4), grd((s->NPYa + 63) / 64, (s->NPXa + 3) / 4);
-  int odd[2] = {0, 0};
-  HIPCHK(hipMemset(s->odd, 0, sizeof odd));
+  StreamMap m[2];
+  for (StreamMap &x : m) x = StreamMap{0, INT_MAX, -1, INT_MAX, -1};
+  HIPCHK(hipMemcpy(s->map, m, sizeof m, hipMemcpyHostToDevice));
   for (int e = 0; e < 2; e++)
-    if (s->ie[e]) hipLaunchKernelGGL(k_stream_ie, grd, blk, 0, 0, eps[e], s->NPXa, s->NPYa, s->ie[e], s->odd + e);
+    if (s->ie[e]) hipLaunchKernelGGL(k_stream_ie, grd, blk, 0, 0, eps[e], s->NPXa, s->NPYa, s->ie[e], s->map + e);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpy(odd, s->odd, sizeof odd, hipMemcpyDeviceToHost));
-  s->isodd = odd[0] || odd[1];
+  HIPCHK(hipMemcpy(m, s->map, sizeof m, hipMemcpyDeviceToHost));
+  s->seen = StreamMap{m[0].odd | m[1].odd, std::min(m[0].i0, m[1].i0), std::max(m[0].i1, m[1].i1),
+                      std::min(m[0].j0, m[1].j0), std::max(m[0].j1, m[1].j1)};
   return FDTD_OK;
 }
 
@@ -956,30 +974,105 @@ long stream_steps_done(const StreamState *s) { return s->steps; }
 // whether a step with these parameters continues the steps taken so far
 bool stream_follows(const StreamState *s, const fdtd_step_params *p)
 {
-  if (!s->coefs || s->isodd) return false;
+  if (!s->coefs || s->seen.odd) return false;
   if (!s->steps) return true;
   return p->angle_deg == s->angle && p->k == s->k && p->omega == s->omega && p->time == s->time + 1 &&
          (s->d.flavour == FDTD_FLAVOUR_MPI || s->d.mode == FDTD_MODE_TM ||
           (p->dot_x == s->dot[0] && p->dot_y == s->dot[1] && p->use_x == s->use[0] && p->use_y == s->use[1]));
 }
 
-static int set_wave(StreamState *s, const fdtd_step_params *p)
+// the wave of a step (its tables, s->wave, are made when a launch needs them)
+static void take_wave(StreamState *s, const fdtd_step_params *p)
 {
-  if (s->wave && p->angle_deg == s->angle && p->k == s->k && p->omega == s->omega) return FDTD_OK;
-  const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI;
+  if (s->wave && p->angle_deg == s->angle && p->k == s->k && p->omega == s->omega) return;
   const double rad = p->angle_deg * M_PI / 180.0;
   s->cpc = cos(rad) / s->d.c0;
   s->spc = sin(rad) / s->d.c0;
+  s->wave = false;
+  s->angle = p->angle_deg;
+  s->k = p->k;
+  s->omega = p->omega;
+}
+
+static int set_wave(StreamState *s, const fdtd_step_params *p)
+{
+  take_wave(s, p);
+  if (s->wave) return FDTD_OK;
+  const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI;
+  const double rad = p->angle_deg * M_PI / 180.0;
   const double kx = mpi ? cos(rad) * p->k : s->cpc * p->omega, ky = mpi ? sin(rad) * p->k : s->spc * p->omega;
   std::vector<D2> t(s->NPXa + s->NPYa);
   for (int i = 0; i < s->NPXa; i++) t[i] = make_double2(cos((i - s->off) * kx), sin((i - s->off) * kx));
   for (int j = 0; j < s->NPYa; j++) t[s->NPXa + j] = make_double2(cos((j - s->off) * ky), sin((j - s->off) * ky));
   HIPCHK(hipMemcpy(s->exy, t.data(), t.size() * sizeof(D2), hipMemcpyHostToDevice));
   s->wave = true;
-  s->angle = p->angle_deg;
-  s->k = p->k;
-  s->omega = p->omega;
   return FDTD_OK;
+}
+
+// the components that carry the pulse, and its projection on them
+static void take_dot(StreamState *s, const fdtd_step_params *p)
+{
+  if (s->d.flavour == FDTD_FLAVOUR_MPI) return;
+  const bool tm = s->d.mode == FDTD_MODE_TM;
+  s->dot[0] = tm ? 1.0 : p->dot_x;
+  s->dot[1] = tm ? 0.0 : p->dot_y;
+  s->use[0] = tm ? 1 : p->use_x;
+  s->use[1] = tm ? 0 : p->use_y;
+}
+
+// the source terms of step e
+static void take_source(StreamState *s, const fdtd_step_params &e)
+{
+  const fdtd_grid_desc &d = s->d;
+  const bool tm = d.mode == FDTD_MODE_TM;
+  if (d.flavour == FDTD_FLAVOUR_MPI) {
+    const double wt = e.omega * e.time;
+    s->c[0] = make_double2(e.ray_coef * cos(wt), -e.ray_coef * sin(wt));
+  } else {
+    // field_scatteredPulse constants (field.c:226-241)
+    const double gx[2] = {tm ? 0.0 : 0.5, 0.0}, gy[2] = {0.0, tm ? 0.0 : 0.5};
+    for (int v = 0; v < 2; v++) {
+      const double t0 = -((d.N_PX / 2.0 + gx[v]) * s->cpc + (d.N_PY / 2 + gy[v]) * s->spc) + 500;
+      s->po[v] = gx[v] * s->cpc + gy[v] * s->spc - (e.time - t0);
+      const double ph = s->po[v] * e.omega;
+      s->c[v] = make_double2(s->dot[v] * cos(ph), s->dot[v] * sin(ph));
+    }
+  }
+  s->ps = make_double2(e.ps_re, e.ps_im);
+}
+
+int stream_note(StreamState *s, const fdtd_step_params *p)
+{
+  take_wave(s, p);
+  take_dot(s, p);
+  take_source(s, *p);
+  s->steps++;
+  s->time = p->time;
+  return FDTD_OK;
+}
+
+// A block takes nearly the same time for any number of steps (its rows pass through every
+// wavefront), the kernels of a step, two launches and with the per-step NTFF two more, as
+// many times as there are steps.  Both in us, fitted to calls of 1 to 9 steps on 40 x 40 to
+// 3200 x 3200 cells.  One step / a block of four: 80 x 80 MPI TM 6.6 / 30, plain TM 6.9 / 35,
+// plain TE 7.3 / 32; 276 x 276 8.6 / 30, 8.5 / 41, 9.0 / 39; 700 x 700 26 / 36, 26 / 52,
+// 26 / 72; 1056 x 1056 53 / 62, 53 / 107, 54 / 97; 2000 x 2000 258 / 153, 268 / 221, 267 / 276;
+// with the per-step NTFF, MPI TM: 80 x 80 16 / 48, 276 x 276 21 / 49, 700 x 700 48 / 75.
+// Calls of three steps so, against a block each: 80 x 80 plain TE 20 / 31, 531 x 402 plain
+// TM 42 / 44, MPI TM 276 x 276 25 / 30.  Frame strips with a scatterer, which form its wave
+// without room to keep it, make a small grid's launch longer: 80 x 80 and 276 x 276 with a
+// cylinder up to the UPML, 8 steps: MPI TM 45, plain TM 56, plain TE 84.
+int stream_few(const StreamState *s, int binned)
+{
+  const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI, tm = s->d.mode == FDTD_MODE_TM;
+  const double n = (double)s->ncell;
+  const double step = 6.5 + 36e-6 * n + 34e-6 * std::max(0.0, n - 9e5) + (binned ? 8 + 5.5e-3 * binned : 0);
+  double launch = (mpi ? 29 + 18e-6 * n : tm ? 40 + 16e-6 * n : 35 + 52e-6 * n) + (binned ? 13 : 0);
+  const StreamMap &m = s->seen;
+  const int h = 2 * STREAM_T;  // a frame strip reaches that far into the box
+  const bool frame = m.i0 < s->xlo + h || m.i1 >= s->xhi - h || m.j0 < s->ylo + h || m.j1 >= s->yhi - h;
+  if (m.i1 >= 0 && frame && n < 262144) launch += mpi ? 16 : tm ? 14 : 45;
+  return std::min(STREAM_T, (int)(launch / step));
 }
 
 static void fill_args(const StreamState *s, StreamArgs &a, const D2 *src, D2 *dst)
@@ -1044,35 +1137,15 @@ static void launch(const StreamState *s, StreamArgs a)
 int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int at, D2 **smp)
 {
   if (n < 1 || n > STREAM_T) return fdtd_fail(FDTD_EINVAL, "bad number of steps %d", n);
-  int rc;
-  const fdtd_grid_desc &d = s->d;
-  const bool mpi = d.flavour == FDTD_FLAVOUR_MPI, tm = d.mode == FDTD_MODE_TM;
-  if ((rc = set_wave(s, p))) return rc;
-  if (!mpi) {
-    s->dot[0] = tm ? 1.0 : p->dot_x;
-    s->dot[1] = tm ? 0.0 : p->dot_y;
-    s->use[0] = tm ? 1 : p->use_x;
-    s->use[1] = tm ? 0 : p->use_y;
-  }
+  const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI, tm = s->d.mode == FDTD_MODE_TM;
+  int rc = set_wave(s, p);
+  if (rc) return rc;
+  take_dot(s, p);
   StreamArgs a;
   fill_args(s, a, *F, s->G);
   a.T = n;
   for (int q = 0; q < n; q++) {
-    const fdtd_step_params &e = p[q];
-    if (mpi) {
-      const double wt = e.omega * e.time;
-      s->c[0] = make_double2(e.ray_coef * cos(wt), -e.ray_coef * sin(wt));
-    } else {
-      // field_scatteredPulse constants (field.c:226-241)
-      const double gx[2] = {tm ? 0.0 : 0.5, 0.0}, gy[2] = {0.0, tm ? 0.0 : 0.5};
-      for (int v = 0; v < 2; v++) {
-        const double t0 = -((d.N_PX / 2.0 + gx[v]) * s->cpc + (d.N_PY / 2 + gy[v]) * s->spc) + 500;
-        s->po[v] = gx[v] * s->cpc + gy[v] * s->spc - (e.time - t0);
-        const double ph = s->po[v] * e.omega;
-        s->c[v] = make_double2(s->dot[v] * cos(ph), s->dot[v] * sin(ph));
-      }
-    }
-    s->ps = make_double2(e.ps_re, e.ps_im);
+    take_source(s, p[q]);
     for (int v = 0; v < 2; v++) {
       a.c[v][q + 1][0] = s->c[v].x;
       a.c[v][q + 1][1] = s->c[v].y;

@@ -444,6 +444,18 @@ int split_set_ns(SplitState *s, const double *nsc, double r2)
 
 int split_depth(const SplitState *s) { return s->coefs && s->cells ? sp_t(s->ph) : 0; }
 
+// Steps that take no more time one by one: a launch of blocks costs nearly the same for
+// any number of them, the kernels of a step, two launches, once a step.  Calls of 1, 2 and
+// 3 steps, one by one / in a block, us: 80 x 80 NS TM 6.1, 12, 19 / 17, 22, 22; 276 x 276
+// split TM 7.5, 15, 22 / 16, 18, 18, NS TE 7.8, 16, 23 / 18, 18, 18; 700 x 700 split TM 18,
+// 36 / 24, 29; 2000 x 2000 split TM 144, 289 / 187, 189, NS TE 220, 439 / 251, 247;
+// 3200 x 3200 split TM 431 / 417, NS TE 529 / 521.
+int split_few(const SplitState *s)
+{
+  const size_t n = s->ncell;
+  return n < (size_t)1 << 16 && s->ph == NS_TM ? 3 : n < (size_t)1 << 18 ? 2 : n < (size_t)8 << 20 ? 1 : 0;
+}
+
 // n <= split_depth() steps of one wave direction from *F, which then holds the new state
 int split_steps(SplitState *s, D2 **F, const fdtd_step_params *p, int n)
 {
