@@ -373,25 +373,30 @@ static fdtd_step_params step_params(int kind)
   return p;
 }
 
+/* n steps were taken, the last at `time`, none past the next check: the check if it is due */
+static void finite_steps(solver_t *s, int n, double time)
+{
+  if ((finite_since_ += n) < finite_every_) return;
+  finite_since_ = 0;
+  long long c[3];
+  CHECK(fdtd_hip_grid_count_nonfinite(s->g, c));
+  const long long cnt = c[0] + c[1] + c[2];
+  if (cnt > 0 && finite_step_ < 0) {
+    finite_step_ = (int)time;
+    finite_count_ = cnt;
+    printf("mpifdtd_amd: %lld non-finite field values after the step of time %d\n", cnt, finite_step_);
+    fflush(stdout);
+    if (finite_abort_) exit(2);
+  }
+}
+
 static void solver_update(int kind)
 {
   solver_t *s = &slv_[kind];
   if (!s->g) { fprintf(stderr, "mpifdtd_amd: update before init\n"); exit(2); }
   const fdtd_step_params p = step_params(kind);
   CHECK(fdtd_hip_grid_step(s->g, &p));
-  if (finite_every_ > 0 && ++finite_since_ >= finite_every_) {
-    finite_since_ = 0;
-    long long c[3];
-    CHECK(fdtd_hip_grid_count_nonfinite(s->g, c));
-    const long long n = c[0] + c[1] + c[2];
-    if (n > 0 && finite_step_ < 0) {
-      finite_step_ = (int)p.time;
-      finite_count_ = n;
-      printf("mpifdtd_amd: %lld non-finite field values after the step of time %d\n", n, finite_step_);
-      fflush(stdout);
-      if (finite_abort_) exit(2);
-    }
-  }
+  if (finite_every_ > 0) finite_steps(s, 1, p.time);
 }
 
 static double complex *solver_field(int kind, int q)
@@ -652,19 +657,21 @@ int fdtd_solver_dims(int out[4])
 static int kind_of(fdtd_method update);
 
 /* up to n steps of the solver that `update` belongs to, field_nextStep after each,
-   handed to the device together; returns how many were taken, 0 where the caller
-   has to step (a finite check runs between steps) */
+   handed to the device together, to the next finite check at most; returns how many
+   were taken, 0 where the caller has to step */
 int solver_run(fdtd_method update, int n)
 {
   const int kind = kind_of(update);
-  if (kind < 0 || !slv_[kind].g || finite_every_ > 0) return 0;
+  if (kind < 0 || !slv_[kind].g) return 0;
   fdtd_step_params p[RUN_STEPS];
   if (n > RUN_STEPS) n = RUN_STEPS;
+  if (finite_every_ > 0 && n > finite_every_ - finite_since_) n = finite_every_ - finite_since_;
   for (int i = 0; i < n; i++) {
     p[i] = step_params(kind);
     field_nextStep();
   }
   CHECK(fdtd_hip_grid_steps(slv_[kind].g, p, n));
+  if (finite_every_ > 0) finite_steps(&slv_[kind], n, p[n - 1].time);
   return n;
 }
 
