@@ -1714,6 +1714,13 @@ __global__ __launch_bounds__(256) void k_bin_records(const double *ts, Contour c
   }
 }
 
+// a device block given back at the end of its scope (dev_free waits for the kernels that use it)
+template <class T>
+struct DevTmp {
+  T *p = nullptr;
+  ~DevTmp() { (void)dev_free(p); }
+};
+
 // bounds of the contour's time shifts over the angles (without their rounding)
 static void shift_span(const fdtd_grid *g, double &lo, double &hi)
 {
@@ -1746,20 +1753,18 @@ static int build_bin_groups(fdtd_grid *g)
   HIPCHK(dev_malloc(&g->binPart, maxp * sizeof(BinPart)));
   HIPCHK(dev_malloc(&g->binRec, maxr * sizeof(BinRec)));
   HIPCHK(hipMemsetAsync(g->binRec, 0xff, maxr * sizeof(BinRec), 0));
-  double *ts = nullptr;
-  int *ctr = nullptr;
-  HIPCHK(dev_malloc(&ts, (size_t)360 * P * sizeof(double)));
-  HIPCHK(dev_malloc(&ctr, 2 * sizeof(int)));
-  HIPCHK(hipMemsetAsync(ctr, 0, 2 * sizeof(int), 0));
-  int rc = time_shifts(g, ts);
+  DevTmp<double> ts;
+  DevTmp<int> ctr;
+  HIPCHK(dev_malloc(&ts.p, (size_t)360 * P * sizeof(double)));
+  HIPCHK(dev_malloc(&ctr.p, 2 * sizeof(int)));
+  HIPCHK(hipMemsetAsync(ctr.p, 0, 2 * sizeof(int), 0));
+  int rc = time_shifts(g, ts.p);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_bin_records, dim3(360, 3), dim3(256), 0, 0, ts, g->ct, nb, g->binPart, g->binRec, ctr);
+  hipLaunchKernelGGL(k_bin_records, dim3(360, 3), dim3(256), 0, 0, ts.p, g->ct, nb, g->binPart, g->binRec, ctr.p);
   HIPCHK(hipGetLastError());
   int n[2] = {0, 0};
-  HIPCHK(hipMemcpy(n, ctr, sizeof n, hipMemcpyDeviceToHost));
+  HIPCHK(hipMemcpy(n, ctr.p, sizeof n, hipMemcpyDeviceToHost));
   g->nparts = n[0];
-  HIPCHK(dev_free(ts));
-  HIPCHK(dev_free(ctr));
   return FDTD_OK;
 }
 
@@ -2278,15 +2283,14 @@ extern "C" int fdtd_hip_grid_form_ns_coefs(fdtd_grid *g, const double *const sig
   if (!g || !sig || !sig[0] || !sig[1] || !sig[2] || !sig[3]) return fdtd_fail(FDTD_EINVAL, "null argument");
   if (g->d.flavour != FDTD_FLAVOUR_NS) return fdtd_fail(FDTD_EINVAL, "per-cell NS coefficients need the NS flavour");
   const int nx = g->d.N_PX, ny = g->d.N_PY;
-  double *t = nullptr;
-  HIPCHK(dev_malloc(&t, 2 * (size_t)(nx + ny) * sizeof(double)));
-  double *const at[4] = {t, t + nx, t + 2 * nx, t + 2 * nx + ny};
+  DevTmp<double> t;
+  HIPCHK(dev_malloc(&t.p, 2 * (size_t)(nx + ny) * sizeof(double)));
+  double *const at[4] = {t.p, t.p + nx, t.p + 2 * nx, t.p + 2 * nx + ny};
   for (int q = 0; q < 4; q++)
     HIPCHK(hipMemcpy(at[q], sig[q], (size_t)(q < 2 ? nx : ny) * sizeof(double), hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_ns_form, dim3((ny + 63) / 64, (nx + 3) / 4), dim3(64, 4), 0, 0, g->eps[0], g->eps[1], g->eps[2], at[0],
                      at[1], at[2], at[3], g->d.mode == FDTD_MODE_TM ? 1 : 0, nx, ny, g->d.mu0, omega, k, g->nsc);
   HIPCHK(hipGetLastError());
-  HIPCHK(dev_free(t));
   g->ns_r2 = r_half;
   if (g->sp) return split_set_ns(g->sp, g->nsc, r_half);
   return FDTD_OK;
@@ -2545,6 +2549,10 @@ extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int 
         m++;
       }
       rc = m > few ? stream_block(g, p + i, m) : FDTD_OK;
+      if (rc == FDTD_ENOMEM) {  // no room for the contour's samples: nothing was launched
+        rc = go_general(g, false);
+        few = m;
+      }
     } else {
       rc = g->st && !g->general ? go_general(g, false) : FDTD_OK;
     }
@@ -2826,9 +2834,14 @@ extern "C" int fdtd_hip_grid_set_dft(fdtd_grid *g, const double *omega, int nf)
   shift_span(g, lo, hi);
   g->dftMlo = (int)floor(lo + g->d.rf_per_c) - 4;
   g->dftNm = (int)ceil(hi + g->d.rf_per_c) + 5 - g->dftMlo;
-  HIPCHK(dev_malloc(&g->dftShift, (size_t)nf * g->dftNm * sizeof(double2)));
-  hipLaunchKernelGGL(k_dft_shift, dim3((g->dftNm + 255) / 256, nf), dim3(256), 0, 0, g->dftOmega, g->dftMlo, g->dftNm,
-                     g->dftShift);
+  if (dev_malloc(&g->dftShift, (size_t)nf * g->dftNm * sizeof(double2)) == hipSuccess) {
+    hipLaunchKernelGGL(k_dft_shift, dim3((g->dftNm + 255) / 256, nf), dim3(256), 0, 0, g->dftOmega, g->dftMlo, g->dftNm,
+                       g->dftShift);
+  } else {  // no room for the table: k_dft_far forms the phases itself
+    (void)hipGetLastError();
+    g->dftShift = nullptr;
+    g->dftNm = 0;
+  }
   HIPCHK(hipGetLastError());
   g->nf = nf;
   // the FP32 fused kernel samples the contour after every inner step

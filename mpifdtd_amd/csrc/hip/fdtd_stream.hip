@@ -787,15 +787,15 @@ int stream_create(const fdtd_grid_desc &d, int off, const Contour &ct, StreamSta
   bool room = dev_malloc(&s->G, 9 * s->stride) == hipSuccess;
   for (int e = 0; e < (d.mode == FDTD_MODE_TM ? 1 : 2); e++)
     room = room && dev_malloc(&s->ie[e], s->ncell * sizeof(double)) == hipSuccess;
+  room = room && dev_malloc(&s->xt, (size_t)s->NPXa * 8 * sizeof(double)) == hipSuccess &&
+         dev_malloc(&s->yt, (size_t)s->NPYa * 6 * sizeof(double)) == hipSuccess &&
+         dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)) == hipSuccess &&
+         dev_malloc(&s->map, 2 * sizeof(StreamMap)) == hipSuccess;
   if (!room) {
     (void)hipGetLastError();
     return FDTD_ENOMEM;
   }
   HIPCHK(hipMemsetAsync(s->G, 0, 9 * s->stride, 0));
-  HIPCHK(dev_malloc(&s->xt, (size_t)s->NPXa * 8 * sizeof(double)));
-  HIPCHK(dev_malloc(&s->yt, (size_t)s->NPYa * 6 * sizeof(double)));
-  HIPCHK(dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)));
-  HIPCHK(dev_malloc(&s->map, 2 * sizeof(StreamMap)));
   s->ctot = ct.total;
   for (int q = 0; q < 4; q++) {
     const Seg &g = ct.s[q];
@@ -946,7 +946,11 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   vf.insert(vf.end(), vi.begin(), vi.end());  // the longer strips first
   (void)dev_free(s->strips);
   s->strips = nullptr;
-  HIPCHK(dev_malloc(&s->strips, vf.size() * sizeof(StreamStrip)));
+  s->coefs = false;
+  if (dev_malloc(&s->strips, vf.size() * sizeof(StreamStrip)) != hipSuccess) {  // the grid steps in place
+    (void)hipGetLastError();
+    return FDTD_OK;
+  }
   HIPCHK(hipMemcpy(s->strips, vf.data(), vf.size() * sizeof(StreamStrip), hipMemcpyHostToDevice));
   s->coefs = true;
   s->wave = false;
@@ -1133,11 +1137,22 @@ static void launch(const StreamState *s, StreamArgs a)
 // n <= STREAM_T steps from the arrays *F, which then hold the new state (the
 // buffer is swapped with the state's own); with at >= 0, the contour's samples
 // after every step in the entries [at, at + n) of the state's STREAM_SAMPLES, from
-// *smp on ([n][3][total])
+// *smp on ([n][3][total]).  FDTD_ENOMEM, with nothing changed, if there is no room for these
 int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int at, D2 **smp)
 {
   if (n < 1 || n > STREAM_T) return fdtd_fail(FDTD_EINVAL, "bad number of steps %d", n);
   const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI, tm = s->d.mode == FDTD_MODE_TM;
+  const size_t entry = 3 * (size_t)s->ctot;
+  if (at >= 0) {
+    if (at + n > STREAM_SAMPLES) return fdtd_fail(FDTD_EINVAL, "bad sample entry %d", at);
+    if (!s->csamp) {
+      if (dev_malloc(&s->csamp, STREAM_SAMPLES * entry * sizeof(D2)) != hipSuccess) {
+        (void)hipGetLastError();
+        return FDTD_ENOMEM;
+      }
+      HIPCHK(hipMemset(s->csamp, 0, STREAM_SAMPLES * entry * sizeof(D2)));
+    }
+  }
   int rc = set_wave(s, p);
   if (rc) return rc;
   take_dot(s, p);
@@ -1155,13 +1170,7 @@ int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int a
     a.ps[q + 1][1] = s->ps.y;
   }
   if (at >= 0) {
-    if (at + n > STREAM_SAMPLES) return fdtd_fail(FDTD_EINVAL, "bad sample entry %d", at);
-    const size_t e = 3 * (size_t)s->ctot;
-    if (!s->csamp) {
-      HIPCHK(dev_malloc(&s->csamp, STREAM_SAMPLES * e * sizeof(D2)));
-      HIPCHK(hipMemset(s->csamp, 0, STREAM_SAMPLES * e * sizeof(D2)));
-    }
-    a.csamp = s->csamp + at * e;
+    a.csamp = s->csamp + at * entry;
     a.ctot = s->ctot;
     memcpy(a.side, s->side, sizeof a.side);
     if (smp) *smp = a.csamp;

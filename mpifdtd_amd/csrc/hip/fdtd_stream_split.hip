@@ -343,14 +343,14 @@ int split_create(const fdtd_grid_desc &d, SplitState **out)
   // a grid without room for a second state, or past 32-bit cell indexes, steps in place
   if (s->ncell >= (size_t)1 << 31) return FDTD_ENOMEM;
   if (dev_malloc(&s->G, 9 * s->stride) != hipSuccess ||
-      dev_malloc(&s->cm, sp_ni(s->ph) * s->ncell * sizeof(double)) != hipSuccess) {
+      dev_malloc(&s->cm, sp_ni(s->ph) * s->ncell * sizeof(double)) != hipSuccess ||
+      dev_malloc(&s->xt, (size_t)s->NPXa * 4 * sizeof(double)) != hipSuccess ||
+      dev_malloc(&s->yt, (size_t)s->NPYa * 3 * sizeof(double)) != hipSuccess ||
+      dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)) != hipSuccess) {
     (void)hipGetLastError();
     return FDTD_ENOMEM;
   }
   HIPCHK(hipMemsetAsync(s->G, 0, 9 * s->stride, 0));
-  HIPCHK(dev_malloc(&s->xt, (size_t)s->NPXa * 4 * sizeof(double)));
-  HIPCHK(dev_malloc(&s->yt, (size_t)s->NPYa * 3 * sizeof(double)));
-  HIPCHK(dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)));
   // Strips: a halo of T cells below and left, T + 1 above and right (the non-standard TE
   // half reaches one cell further there).  Rows per strip as in fdtd_stream.hip: the
   // shortest strips that all run at once, two workgroups on each of 256 compute units.
@@ -375,7 +375,10 @@ int split_create(const fdtd_grid_desc &d, SplitState **out)
     if (v.size() <= 512) break;
   }
   s->ns = (int)v.size();
-  HIPCHK(dev_malloc(&s->strips, v.size() * sizeof(SplitStrip)));
+  if (dev_malloc(&s->strips, v.size() * sizeof(SplitStrip)) != hipSuccess) {
+    (void)hipGetLastError();
+    return FDTD_ENOMEM;
+  }
   HIPCHK(hipMemcpy(s->strips, v.data(), v.size() * sizeof(SplitStrip), hipMemcpyHostToDevice));
   return FDTD_OK;
 }
