@@ -209,9 +209,9 @@ int fdtd_hip_grid_sync(fdtd_grid *g);
 int fdtd_hip_grid_set_blocking(fdtd_grid *g, int T, int R);
 int fdtd_hip_grid_get_blocking(const fdtd_grid *g, int *T, int *R);
 /* FP32 grids: how a block's UPML and interior tiles are launched.  AUTO picks
- * MERGED for small grids (plain TE: TWO_STREAMS_P16) and SPLIT_P16 from 0.8 (TE), 1
- * (plain TM; 2 with the per-step NTFF) or 4 (MPI TM; 1 with the running DFT alone)
- * million cells; MERGED is one launch of both
+ * MERGED for small grids and shallow blocks, else SPLIT_P16 (plain TE also
+ * TWO_STREAMS_P16, short interior tiles SPLIT), by the solver, the grid's size, the
+ * blocking and what samples the contour; MERGED is one launch of both
  * (one register budget, the UPML body's); SPLIT is two launches in a row, each
  * at its own occupancy; TWO_STREAMS runs the two launches side by side on two
  * streams. */

@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -1693,26 +1694,81 @@ static int update_wave(FastState *s, const fdtd_step_params &p)
   return FDTD_OK;
 }
 
-// The launch shape of FAST_LAUNCH_AUTO: one merged launch while the tiles leave the
-// chip partly idle, the two kinds apart with 8- and 16-wavefront tiles once each
-// fills it; the plain TE body, which spills at the merged kernel's budget, beside each
-// other on two streams instead.  The lines lie between the sizes timed (8-step blocks,
-// R = 16, us; merged / SPLIT_P16 / TWO_STREAMS_P16 on 500 x 400, 1056 x 1056 and
-// 2000 x 1500 cells): MPI TM 24/36/44, 34/43/54, 59/62/74; MPI TE 25/39/45, 53/48/57,
-// 100/72/83; plain TM 34/47/43, 51/50/58, 76/69/79; plain TE 60/66/46, 91/65/72,
-// 148/86/95.  The former two-launch shape of large grids
-// (SPLIT, 4-wavefront tiles) took 71, 93, 88 and 137 on 2000 x 1500.  The binning of the
-// per-step NTFF beside the launches moves plain TM's line up (76/89 on 1056 x 1056, 91/104
-// on 1300 x 1200, 127/123 on 1600 x 1400; merged / SPLIT_P16), the running DFT alone, which
-// needs little of the chip, MPI TM's down (47/47 on 800 x 800, 57/52, 67/61, 72/68).
+// The launch shape of FAST_LAUNCH_AUTO.  One merged launch while the tiles leave the chip
+// partly idle; beyond that the two kinds apart, each at its own register budget: with 8- and
+// 16-wavefront tiles (SPLIT_P16), as 4-wavefront tiles where the interior ones are short
+// (SPLIT), or, plain TE, whose body spills at the merged kernel's budget, beside each other
+// on two streams (TWO_STREAMS_P16).  Which grid is large enough depends on the work of a
+// launch: shallow blocks are short, and a second launch costs them more (plain TE on
+// 80 x 80, us per step, MERGED / TWO_STREAMS_P16: T = 1 13 / 36, T = 4 6.7 / 11, T = 10
+// 5.4 / 5.7).  Lines from all four shapes timed on 80 x 80 to 5240 x 5160 cells, 1140 runs,
+// in which they take 0.3 % more than the fastest shape on average, 14 % at worst.  Some of
+// them, us per step, MERGED / SPLIT / SPLIT_P16 / TWO_STREAMS_P16, R = 16: MPI TM
+// 1056 x 1056, T = 8 4.2 / 5.9 / 5.3 / 6.7, 3000 x 2400 16.4 / 17.4 / 18.8 / 19.7; plain TM
+// 1056 x 1056, T = 4 6.7 / 10.8 / 9.3 / 10.9, T = 10 6.8 / 8.4 / 6.4 / 6.2; MPI TE
+// 1056 x 1056, T = 1 18.5 / 26.1 / 28.0 / 40.5, T = 8 6.6 / 6.1 / 5.9 / 7.2; plain TE
+// 2000 x 1500, T = 4 20.1 / 18.1 / 15.1 / 16.5, T = 8 19.5 / 17.4 / 10.9 / 12.3.
+struct AutoLines {
+  int R, T;                // for at least these rows per wavefront and steps per block
+  int p16[4], split[4];    // Ki cells from which SPLIT_P16 / SPLIT runs: MPI TM, plain TM, MPI TE, plain TE
+  int two;                 // plain TE: below p16, TWO_STREAMS_P16 from here on
+};
+enum { AUTO_NO = INT_MAX };
+#define AUTO_NONE {AUTO_NO, AUTO_NO, AUTO_NO, AUTO_NO}
+static const AutoLines auto_lines[] = {
+    {16, 12, {1536, 512, 448, 448}, AUTO_NONE, 16},
+    {16, 10, {16384, 768, 704, 704}, AUTO_NONE, 24},
+    {16, 8, {16384, 960, 896, 768}, AUTO_NONE, 24},
+    {16, 7, {AUTO_NO, AUTO_NO, 1792, 600}, AUTO_NONE, 64},
+    {16, 6, {AUTO_NO, AUTO_NO, 1792, 512}, AUTO_NONE, 448},
+    {16, 5, {AUTO_NO, AUTO_NO, 1280, 704}, AUTO_NONE, AUTO_NO},
+    {16, 3, {AUTO_NO, AUTO_NO, AUTO_NO, 896}, {AUTO_NO, AUTO_NO, 2560, AUTO_NO}, AUTO_NO},
+    {16, 2, {AUTO_NO, AUTO_NO, AUTO_NO, 2560}, {AUTO_NO, AUTO_NO, 8192, AUTO_NO}, AUTO_NO},
+    {16, 1, AUTO_NONE, AUTO_NONE, AUTO_NO},
+    {8, 8, {3072, 1792, 896, 320}, {6144, 6144, 6144, 6144}, AUTO_NO},
+    {8, 6, {AUTO_NO, 3072, 1152, 640}, {6144, 6144, 6144, 6144}, AUTO_NO},
+    {8, 3, {AUTO_NO, AUTO_NO, 2048, 960}, {9216, 9216, 9216, 9216}, AUTO_NO},
+    {8, 2, {AUTO_NO, AUTO_NO, AUTO_NO, 1792}, {AUTO_NO, AUTO_NO, 4096, AUTO_NO}, AUTO_NO},
+    {8, 1, AUTO_NONE, {AUTO_NO, AUTO_NO, 5120, 4096}, AUTO_NO},
+    {0, 2, AUTO_NONE, {6144, 6144, 1280, 896}, AUTO_NO},
+    {0, 0, AUTO_NONE, {6144, 6144, 1536, 1280}, AUTO_NO},
+};
+
 static int auto_shape(const FastState *s)
 {
-  const size_t cells = (size_t)s->h.NPX * s->h.NPY;
+  const int ki = (int)std::min<size_t>((size_t)s->h.NPX * s->h.NPY >> 10, INT_MAX - 1);
   const bool tm = s->d.mode == FDTD_MODE_TM, mpi = s->d.flavour == FDTD_FLAVOUR_MPI;
   const bool dft = s->csamp && !s->binned, bin = s->csamp && s->binned;
-  const size_t line = !tm ? (size_t)3 << 18 : mpi ? (size_t)(dft ? 1 : 4) << 20 : (size_t)(bin ? 2 : 1) << 20;
-  if (cells >= line) return FAST_LAUNCH_SPLIT_P16;
-  return tm || mpi ? FAST_LAUNCH_MERGED : FAST_LAUNCH_TWO_STREAMS_P16;
+  const AutoLines *l = auto_lines;
+  while (s->R < l->R || s->T < l->T) l++;
+  const int q = (tm ? 0 : 2) + (mpi ? 0 : 1);
+  int p16 = l->p16[q], split = l->split[q], two = tm || mpi ? AUTO_NO : l->two;
+  if (s->R >= 16 && s->T >= 8) {
+    // The running DFT alone, which needs little of the chip, moves TM's lines down (MPI TM
+    // 1056 x 1056, T = 8, MERGED / SPLIT_P16 7.2 / 6.6), the per-step NTFF's binning beside
+    // the launches moves plain TM's up (1056 x 1056 9.8 / 11.5, 1840 x 1760 21.3 / 21.1) and
+    // plain TE's (640 x 560 MERGED / TWO_STREAMS_P16 9.0 / 9.8).
+    if (tm && dft) p16 = std::min(p16, 960);
+    if (tm && !mpi && bin) p16 = std::max(p16, 2048);
+    if (bin) two = std::max(two, 512);
+    // plain TM at T = 8: 2640 x 2560 MERGED / SPLIT_P16 17.6 / 19.3; 2 to 6 % the other way on either side
+    if (tm && !mpi && !s->csamp && s->T < 10 && ki >= 5120 && ki < 16384) return FAST_LAUNCH_MERGED;
+  }
+  if (s->R >= 16 && s->T < 6 && s->csamp && !tm) {
+    // shallow blocks with samples, T = 4: MPI TE 2040 x 1960 MERGED / SPLIT_P16 28.5 / 20.6 (DFT),
+    // 37.2 / 29.6 (NTFF), 1640 x 1560 22.3 / 21.4 (NTFF); plain TE with the DFT 1040 x 960
+    // MERGED / SPLIT_P16 / TWO_STREAMS_P16 15.6 / 16.1 / 13.3
+    if (mpi && s->T >= 3) {
+      p16 = dft ? 1792 : 2304;
+      split = AUTO_NO;
+    } else if (!mpi) {
+      if (dft && s->T >= 3) return ki >= 600 ? FAST_LAUNCH_TWO_STREAMS_P16 : FAST_LAUNCH_MERGED;
+      p16 = std::max(p16, 2304);
+    }
+  }
+  if (ki >= split) return FAST_LAUNCH_SPLIT;
+  if (ki >= p16) return FAST_LAUNCH_SPLIT_P16;
+  return ki >= two ? FAST_LAUNCH_TWO_STREAMS_P16 : FAST_LAUNCH_MERGED;
 }
 
 // The samples of the blocks launched since the last call to the consumer (NTFF).
