@@ -283,7 +283,9 @@ int fdtd_hip_batch_run(fdtd_hip_batch *b, int blocks);
  * side on two streams (FAST_LAUNCH_TWO_STREAMS).  The *_PML8 and *_W8 shapes run
  * wide UPML tiles (48 rows as 16 wavefronts), all of them but SPLIT_PML8 the
  * interior tiles as 8 wavefronts (R >= 8), and the two on two streams the TE
- * instances beside the TM ones.  Default: FAST_LAUNCH_TWO_STREAMS_PML8. */
+ * instances beside the TM ones.  The two on two streams run
+ * a batch of one mode whose tiles nearly all run at once, or with R = 4 and many interior
+ * tiles, as 32-row UPML tiles of 8 wavefronts beside 4-wavefront interior tiles.  Default: FAST_LAUNCH_TWO_STREAMS_PML8. */
 int fdtd_hip_batch_set_launch_mode(fdtd_hip_batch *b, int mode);
 int fdtd_hip_batch_sync(fdtd_hip_batch *b, int *steps_done);
 int fdtd_hip_batch_destroy(fdtd_hip_batch *b);

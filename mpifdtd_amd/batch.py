@@ -76,7 +76,8 @@ class Batch:
     def set_launch_mode(self, mode):
         """2: interior tiles then UPML tiles; 3: the two side by side on two streams; 4: 2 with wide
         UPML tiles (48 rows as 16 wavefronts); 6: 4 with the interior tiles as 8 wavefronts; 5 (the
-        default) and 7: 6 with the TE instances beside the TM ones on two streams (FAST_LAUNCH_* of
+        default) and 7: 6 with the TE instances beside the TM ones on two streams, or, a batch of one mode
+        that fits the GPU at once, 32-row UPML tiles beside the interior ones (FAST_LAUNCH_* of
         fdtd_hip.h)."""
         check(N.lib().fdtd_batch_set_launch_mode(self._h, int(mode)), "fdtd_batch_set_launch_mode")
 

@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <type_traits>
 #include <climits>
+#include <cstdint>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -895,12 +896,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(fast_interi
 // rows (512 threads), UPML tiles of FAST_UPML_ROWS_WIDE = 48 rows as 16 wavefronts of
 // 3 rows (1024 threads): of a tile's rows 48 - 2T - 1 are core rows where a 32-row tile
 // keeps 32 - 2T - 1 (T = 8: 31 and 15); a block of 32 TM instances of 400 x 400 cells
-// took 285 us with 32-row tiles as 8 wavefronts of 4 rows, 238 with these.
+// took 285 us with 32-row tiles as 8 wavefronts of 4 rows (WIDE = 2, UPML tiles alone),
+// 238 with these.  Where all tiles run at once the shorter ones are the faster
+// (FastBatch::small).
 template <int MODE, int R, int KQ, int WIDE = 0>
-__global__ __launch_bounds__(!WIDE ? 256 : (KQ == 0 ? 1024 : 512))
-__attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(WIDE ? R / 2 : R) : (WIDE ? 4 : 1)))) void k_fast_batch(FastArgs a)
+__global__ __launch_bounds__(!WIDE ? 256 : (KQ == 0 && WIDE == 1 ? 1024 : 512))
+__attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(WIDE ? R / 2 : R) : (WIDE == 1 ? 4 : 1)))) void k_fast_batch(FastArgs a)
 {
   static_assert(!WIDE || (KQ != 2 && R >= 8), "wide bodies: one queue, R >= 8");
+  static_assert(WIDE != 2 || KQ == 0, "32-row tiles as 8 wavefronts: UPML tiles");
   __shared__ int s_tid;
   for (int k = (KQ == 1 ? 1 : 0); k < (KQ == 0 ? 1 : 2); k++) {
     // the queue in 8 contiguous parts, one per XCD (workgroup b runs on XCD b % 8):
@@ -922,7 +926,8 @@ __attribute__((amdgpu_waves_per_eu(KQ == 1 ? fast_interior_waves(WIDE ? R / 2 : 
         continue;
       }
       if constexpr (WIDE) {
-        if (KQ == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, FAST_UPML_ROWS_WIDE / 16, 1, 1, 0, 16>(a, a.qoff[0] + tid);
+        if (KQ == 0 && WIDE == 2) fast_tile<MODE, FDTD_FLAVOUR_MPI, FAST_UPML_ROWS / 8, 1, 1, 0, 8>(a, a.qoff[0] + tid);
+        else if (KQ == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, FAST_UPML_ROWS_WIDE / 16, 1, 1, 0, 16>(a, a.qoff[0] + tid);
         else fast_tile<MODE, FDTD_FLAVOUR_MPI, R / 2, 0, 1, 0, 8>(a, a.qoff[1] + tid);
       } else {
         if (KQ != 1 && k == 0) fast_tile<MODE, FDTD_FLAVOUR_MPI, 8, 1, 1, 0>(a, a.qoff[0] + tid);
@@ -2118,7 +2123,15 @@ struct FastBatch {
   // 4 of them 344 / 340 / 308; 32 TM of 400 x 400 238 / 239 / 238; before (32-row UPML
   // tiles, KINDS) 821, 344 and 288.  Interior tiles as 4 wavefronts beside: 905 us and 339.
   // Default: TWO_STREAMS_PML8 (every shape gives the same bits).
-  int two_streams = BATCH_MODES, wide = 1, inner8 = 0;
+  int two_streams = BATCH_MODES, wide = 1, inner8 = 0, shape = FAST_LAUNCH_TWO_STREAMS_PML8;
+  // TWO_STREAMS_PML8 and _W8 of a batch of one mode, whose launches would follow each other:
+  // the UPML tiles of 32 rows as 8 wavefronts beside 4-wavefront interior tiles (wide = 2)
+  // where nearly all of them run at once, or where the interior tiles are short and many (no
+  // 8-wavefront ones at R = 4).  Per block, us, these / the wide ones apart: R = 16 one
+  // 400 x 400, T = 8 46 / 51, T = 12 58 / 63, four 100 x 100 46 / 51, one 700 x 700 (about 350
+  // tiles) 65 / 66, four 300 x 300 61 / 60, T = 4 eight 200 x 200 (192 UPML tiles) 54 / 49; R = 8 one 400 x 400 54 / 57; R = 4, T = 4 one
+  // 1000 x 1000 99 / 106, one 200 x 200 39.5 / 38.6.  -1: not counted yet
+  int small = -1;
   int tilesU = -1;  // rows of the UPML tiles in dtiles
   hipStream_t s2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -2128,9 +2141,10 @@ struct FastBatch {
 };
 
 template <int MODE, int KQ>
-static void batch_launch_q(const FastArgs &a, int R, int nblk, bool wide, hipStream_t st)
+static void batch_launch_q(const FastArgs &a, int R, int nblk, int wide, hipStream_t st)
 {
-  if (wide && KQ == 0) hipLaunchKernelGGL((k_fast_batch<MODE, 8, 0, 1>), dim3(nblk), dim3(1024), 0, st, a);
+  if (wide == 2 && KQ == 0) hipLaunchKernelGGL((k_fast_batch<MODE, 8, 0, 2>), dim3(nblk), dim3(512), 0, st, a);
+  else if (wide && KQ == 0) hipLaunchKernelGGL((k_fast_batch<MODE, 8, 0, 1>), dim3(nblk), dim3(1024), 0, st, a);
   else if (wide && R == 8) hipLaunchKernelGGL((k_fast_batch<MODE, 8, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
   else if (wide && R == 16) hipLaunchKernelGGL((k_fast_batch<MODE, 16, KQ, 1>), dim3(nblk), dim3(512), 0, st, a);
   else if (R == 4) hipLaunchKernelGGL((k_fast_batch<MODE, 4, KQ>), dim3(nblk), dim3(256), 0, st, a);
@@ -2142,8 +2156,8 @@ template <int MODE>
 static void batch_launch_mode(const FastBatch *b, const FastArgs &a, const int nblk[2], hipStream_t st,
                               hipStream_t st_pml)
 {
-  if (nblk[1] > 0) batch_launch_q<MODE, 1>(a, b->R, nblk[1], b->inner8 != 0, st);
-  if (nblk[0] > 0) batch_launch_q<MODE, 0>(a, b->R, nblk[0], b->wide != 0, st_pml);
+  if (nblk[1] > 0) batch_launch_q<MODE, 1>(a, b->R, nblk[1], b->inner8, st);
+  if (nblk[0] > 0) batch_launch_q<MODE, 0>(a, b->R, nblk[0], b->wide, st_pml);
 }
 
 static FastArgs batch_args(const FastBatch *b, int m)
@@ -2213,33 +2227,62 @@ void fast_batch_destroy(FastBatch *b)
   delete b;
 }
 
+// (with small known: see there)
 static void batch_shape(FastBatch *b, int mode)
 {
+  b->shape = mode;
   b->wide = mode >= FAST_LAUNCH_SPLIT_PML8;
   b->two_streams = mode == FAST_LAUNCH_TWO_STREAMS ? BATCH_KINDS
                    : mode == FAST_LAUNCH_TWO_STREAMS_PML8 || mode == FAST_LAUNCH_TWO_STREAMS_W8 ? BATCH_MODES : 0;
   b->inner8 = b->wide && mode != FAST_LAUNCH_SPLIT_PML8 && b->R >= 8;
+  if (b->small == 1 && b->wide && b->two_streams == BATCH_MODES) {
+    b->wide = 2;
+    b->two_streams = BATCH_KINDS;
+    b->inner8 = 0;
+  }
 }
 
 // The tile queues of the launch shape: per mode, the UPML queue then the interior queue,
 // instances largest first (longest-processing-time order).
 static int batch_tiles(FastBatch *b)
 {
-  const int rows = b->wide ? FAST_UPML_ROWS_WIDE : FAST_UPML_ROWS;
-  if (b->tilesU == rows) return FDTD_OK;
   int rc;
+  // tile lists of UPML tiles of that height, until there are more than `most` tiles
+  auto build = [&](int rows, size_t most, size_t &np, size_t &ni) -> int {
+    np = ni = 0;
+    for (FastState *s : b->st) {
+      // (an instance stepped by itself meanwhile has its own tiles)
+      if ((rc = fast_state_set_blocking(s, b->T, b->R))) return rc;
+      s->upmlRows = rows;
+      if (s->tilesT != s->T || s->tilesR != s->R || s->tilesU != s->upmlRows)
+        if ((rc = build_tiles(s))) return rc;
+      np += s->htp.size();
+      ni += s->hti.size();
+      if (np + ni > most) break;
+    }
+    return FDTD_OK;
+  };
+  size_t np, ni;
+  if (b->small < 0) {
+    bool one = true;
+    for (FastState *s : b->st) one = one && s->d.mode == b->st[0]->d.mode;
+    b->small = 0;
+    if (one) {
+      // nearly at once: two interior tiles, or a UPML one beside an interior one, on each of 256 compute units
+      const size_t all = b->R >= 8 ? 352 : SIZE_MAX;
+      if ((rc = build(FAST_UPML_ROWS, all, np, ni))) return rc;
+      b->small = b->R >= 8 ? np + ni <= all && np <= 168 : ni >= 256;
+    }
+    batch_shape(b, b->shape);
+  }
+  const int rows = b->wide == 1 ? FAST_UPML_ROWS_WIDE : FAST_UPML_ROWS;
+  if (b->tilesU == rows) return FDTD_OK;
+  if ((rc = build(rows, SIZE_MAX, np, ni))) return rc;
   std::vector<int> order(b->n);
   for (int i = 0; i < b->n; i++) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
     return (long)b->st[x]->h.NPX * b->st[x]->h.NPY > (long)b->st[y]->h.NPX * b->st[y]->h.NPY;
   });
-  for (FastState *s : b->st) {
-    // (an instance stepped by itself meanwhile has its own tiles)
-    if ((rc = fast_state_set_blocking(s, b->T, b->R))) return rc;
-    s->upmlRows = rows;
-    if (s->tilesT != s->T || s->tilesR != s->R || s->tilesU != s->upmlRows)
-      if ((rc = build_tiles(s))) return rc;
-  }
   std::vector<FastTile> all;
   int off[2][2], nt[2][2];
   for (int m = 0; m < 2; m++)
@@ -2382,14 +2425,10 @@ int fast_batch_set_launch(FastBatch *b, int mode)
   if (b->graph) (void)hipGraphDestroy(b->graph);
   b->gexec = nullptr;
   b->graph = nullptr;
-  const int old[3] = {b->wide, b->two_streams, b->inner8};
+  const int old = b->shape;
   batch_shape(b, mode);
   const int rc = batch_tiles(b);
-  if (rc) {  // the bodies must match the tiles: keep both as they were
-    b->wide = old[0];
-    b->two_streams = old[1];
-    b->inner8 = old[2];
-  }
+  if (rc) batch_shape(b, old);  // the bodies must match the tiles: keep both as they were
   return rc;
 }
 
