@@ -2616,7 +2616,8 @@ extern "C" int fdtd_hip_grid_reset(fdtd_grid *g)
   int rc0 = ntff_sync(g);
   if (rc0) return rc0;
   g->smpN = 0;
-  for (int f = 0; f < 9; f++)
+  if (g->F64) HIPCHK(hipMemset(g->F64, 0, 9 * stream_stride(g->ncell)));
+  for (int f = 0; f < 9 && !g->F64; f++)
     if (g->F[f]) HIPCHK(hipMemset(g->F[f], 0, g->ncell * sizeof(double2)));
   for (int a = 0; a < 3 && g->ntn; a++) HIPCHK(hipMemset(g->ntb[a], 0, g->ntn * sizeof(double2)));
   if (g->nf) {
