@@ -940,14 +940,17 @@ __global__ __launch_bounds__(256) void k_dft_phase(const double *omega, int nf, 
 // k_dft_shift's table (formed here, per angle, cell and frequency, their sines and cosines
 // were most of the time), and a workgroup's angles share the reads of V: 24.6k contour
 // cells, 81 frequencies 4.5 -> 2.8 ms (what is left: the shifts and V read from beyond the
-// L2 caches).
+// L2 caches).  Few frequencies, which leave the chip idle, take one angle a workgroup
+// (24.6k cells, one frequency 63 -> 46 us a read), short contours, whose reductions count,
+// one of a single wavefront (60 x 60 grid, 81 frequencies 279 -> 145 us).
 #define DFT_FAR_ANG 4
-__global__ __launch_bounds__(256) void k_dft_far(const double2 *VE, const double2 *VH, Contour ct, const double *ts,
+template <int ANG, int NT>
+__global__ __launch_bounds__(NT) void k_dft_far(const double2 *VE, const double2 *VH, Contour ct, const double *ts,
                                                  const double *omega, const double2 *shift, int mlo, int nm, double cf,
                                                  double2 *out)
 {
-  __shared__ double red[DFT_FAR_ANG][6][4];
-  const int ang0 = blockIdx.x * DFT_FAR_ANG, f = blockIdx.y, P = ct.total;
+  __shared__ double red[ANG][6][NT / 64];
+  const int ang0 = blockIdx.x * ANG, f = blockIdx.y, P = ct.total;
   const double w = omega[f];
   const double2 *ph = shift + (size_t)f * nm;
   double sn1, cs1, sn2, cs2;
@@ -955,21 +958,21 @@ __global__ __launch_bounds__(256) void k_dft_far(const double2 *VE, const double
   sincos(2.0 * w, &sn2, &cs2);
   // b + (a - b) e^{iw} - a e^{2iw} with b = 1 - a: c0 + a c1
   const double c0r = 1.0 - cs1, c0i = -sn1, c1r = 2.0 * cs1 - 1.0 - cs2, c1i = 2.0 * sn1 - sn2;
-  double acc[DFT_FAR_ANG][3][2];
+  double acc[ANG][3][2];
 #pragma unroll
-  for (int g = 0; g < DFT_FAR_ANG; g++)
+  for (int g = 0; g < ANG; g++)
 #pragma unroll
     for (int k = 0; k < 6; k++) acc[g][k >> 1][k & 1] = 0.0;
   for (int q = 0; q < 4; q++) {
     // a side's E and H samples go to one array each: the sums choose it once a side
     const int p1 = q < 3 ? ct.s[q + 1].off : P;
-    double sum[2][DFT_FAR_ANG][2];
+    double sum[2][ANG][2];
 #pragma unroll
-    for (int k = 0; k < 4 * DFT_FAR_ANG; k++) sum[k / (2 * DFT_FAR_ANG)][(k >> 1) % DFT_FAR_ANG][k & 1] = 0.0;
-    for (int p = ct.s[q].off + threadIdx.x; p < p1; p += 256) {
+    for (int k = 0; k < 4 * ANG; k++) sum[k / (2 * ANG)][(k >> 1) % ANG][k & 1] = 0.0;
+    for (int p = ct.s[q].off + threadIdx.x; p < p1; p += NT) {
       const double2 ve = VE[(size_t)f * P + p], vh = VH[(size_t)f * P + p];
 #pragma unroll
-      for (int g = 0; g < DFT_FAR_ANG; g++) {
+      for (int g = 0; g < ANG; g++) {
         const double t = ts[(size_t)(ang0 + g) * P + p];
 #pragma unroll
         for (int hh = 0; hh < 2; hh++) {
@@ -991,7 +994,7 @@ __global__ __launch_bounds__(256) void k_dft_far(const double2 *VE, const double
     for (int hh = 0; hh < 2; hh++) {
       const int arr = hh ? ct.s[q].wa : ct.s[q].ua;
 #pragma unroll
-      for (int g = 0; g < DFT_FAR_ANG; g++)
+      for (int g = 0; g < ANG; g++)
 #pragma unroll
         for (int k = 0; k < 6; k++)
           if (k >> 1 == arr) acc[g][k >> 1][k & 1] += sum[hh][g][k & 1];
@@ -999,7 +1002,7 @@ __global__ __launch_bounds__(256) void k_dft_far(const double2 *VE, const double
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
-  for (int g = 0; g < DFT_FAR_ANG; g++)
+  for (int g = 0; g < ANG; g++)
 #pragma unroll
     for (int k = 0; k < 6; k++) {
       double v = acc[g][k >> 1][k & 1];
@@ -1007,10 +1010,10 @@ __global__ __launch_bounds__(256) void k_dft_far(const double2 *VE, const double
       if (lane == 0) red[g][k][wv] = v;
     }
   __syncthreads();
-  if (threadIdx.x < 3 * DFT_FAR_ANG) {
+  if (threadIdx.x < 3 * ANG) {
     const int aa = threadIdx.x % 3, g = threadIdx.x / 3;
     double re = 0.0, im = 0.0;
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < NT / 64; k++) {
       re += red[g][2 * aa][k];
       im += red[g][2 * aa + 1][k];
     }
@@ -2862,8 +2865,10 @@ extern "C" int fdtd_hip_grid_get_dft(fdtd_grid *g, double *out)
   if ((rc = ntff_sync(g))) return rc;
   dft_flush(g, 0);
   const double cf = g->d.flavour == FDTD_FLAVOUR_PLAIN ? 1.0 : g->coef;
-  hipLaunchKernelGGL(k_dft_far, dim3(360 / DFT_FAR_ANG, g->nf), dim3(256), 0, 0, g->dftE, g->dftH, g->ct, g->dftTs,
-                     g->dftOmega, g->dftShift, g->dftMlo, g->dftNm, cf, g->dftOut);
+  const bool brief = g->ct.total < 768, one = brief || g->nf < 4;
+  hipLaunchKernelGGL((brief ? k_dft_far<1, 64> : one ? k_dft_far<1, 256> : k_dft_far<DFT_FAR_ANG, 256>),
+                     dim3(one ? 360 : 360 / DFT_FAR_ANG, g->nf), dim3(brief ? 64 : 256), 0, 0, g->dftE, g->dftH, g->ct,
+                     g->dftTs, g->dftOmega, g->dftShift, g->dftMlo, g->dftNm, cf, g->dftOut);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpy(out, g->dftOut, (size_t)g->nf * 3 * 360 * sizeof(double2), hipMemcpyDeviceToHost));
   return FDTD_OK;
