@@ -2542,6 +2542,10 @@ extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int 
       few = split_few(g->sp);
       while (m < split_depth(g->sp) && i + m < n && p[i + m].angle_deg == a.angle_deg && p[i + m].k == a.k) m++;
       rc = m > few ? split_block(g, p + i, m) : FDTD_OK;
+      if (rc == FDTD_ENOMEM) {  // no room for the second state: nothing was launched
+        rc = go_general(g, false);
+        few = m;
+      }
     } else if (g->st && !g->general && stream_follows(g->st, &a)) {
       few = stream_few(g->st, g->ntn ? g->ct.total : 0);
       while (m < STREAM_T && i + m < n) {
@@ -2552,7 +2556,7 @@ extern "C" int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int 
         m++;
       }
       rc = m > few ? stream_block(g, p + i, m) : FDTD_OK;
-      if (rc == FDTD_ENOMEM) {  // no room for the contour's samples: nothing was launched
+      if (rc == FDTD_ENOMEM) {  // no room for the second state or the contour's samples: nothing was launched
         rc = go_general(g, false);
         few = m;
       }

@@ -716,27 +716,50 @@ __global__ __launch_bounds__(256) void k_stream_aux(StreamArgs a)
 // What the host asks of a permittivity map: whether a cell's 1/eps lies outside
 // [STREAM_IE_MIN, 1 / STREAM_IE_MIN], NaN included, and the box of the scatterer's cells.
 struct StreamMap {
-  int odd, i0, i1, j0, j1;  // rows [i0, i1], columns [j0, j1]
+  int odd, i0, i1, j0, j1;  // rows [NPXa - i0, i1), columns [NPYa - j0, j1): all zero without a scatterer
 };
 
-// 1/eps, 0 on the ring of cells that are never updated
+// 1/eps, 0 on the ring of cells that are never updated.  A workgroup takes 64 columns of
+// STREAM_IE_ROWS rows, so that few wavefronts widen the map's box: with one row each, their
+// accesses to it were most of the time (2000 x 1500 with a cylinder 77 -> 23 us).
+#define STREAM_IE_ROWS 32
 __global__ __launch_bounds__(256) void k_stream_ie(const double *eps, int NPXa, int NPYa, double *ie, StreamMap *m)
 {
-  const int j = blockIdx.x * 64 + threadIdx.x, i = blockIdx.y * 4 + threadIdx.y;
-  const bool in = i < NPXa && j < NPYa, ring = i == 0 || j == 0 || i >= NPXa - 1 || j >= NPYa - 1;
-  const size_t k = (size_t)i * NPYa + j;
-  const double v = in ? 1.0 / eps[k] : 1.0;
-  if (in) ie[k] = ring ? 0.0 : v;
-  if (!ring && !(fabs(v) >= STREAM_IE_MIN && fabs(v) <= 1.0 / STREAM_IE_MIN)) m->odd = 1;
-  // a wavefront holds 64 columns of one row; few of them still widen the box
-  const unsigned long long b = __ballot(!ring && v != 1.0);
-  if (!b || threadIdx.x) return;
-  const int j0 = j + __builtin_ctzll(b), j1 = j + 63 - __builtin_clzll(b);
-  auto now = [](int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  if (i < now(&m->i0)) atomicMin(&m->i0, i);
-  if (i > now(&m->i1)) atomicMax(&m->i1, i);
-  if (j0 < now(&m->j0)) atomicMin(&m->j0, j0);
-  if (j1 > now(&m->j1)) atomicMax(&m->j1, j1);
+  const int j = blockIdx.x * 64 + threadIdx.x, r0 = blockIdx.y * STREAM_IE_ROWS + threadIdx.y;
+  unsigned long long cols = 0;  // of the scatterer's cells, and their rows
+  int lo = INT_MAX, hi = -1;
+  bool odd = false;
+#pragma unroll
+  for (int r = 0; r < STREAM_IE_ROWS; r += 4) {
+    const int i = r0 + r;
+    const bool in = i < NPXa && j < NPYa, ring = i == 0 || j == 0 || i >= NPXa - 1 || j >= NPYa - 1;
+    const size_t k = (size_t)i * NPYa + j;
+    const double v = in ? 1.0 / eps[k] : 1.0;
+    if (in) ie[k] = ring ? 0.0 : v;
+    odd = odd || (!ring && !(fabs(v) >= STREAM_IE_MIN && fabs(v) <= 1.0 / STREAM_IE_MIN));
+    const unsigned long long b = __ballot(!ring && v != 1.0);
+    cols |= b;
+    if (b) {
+      lo = min(lo, i);
+      hi = i;
+    }
+  }
+  if (odd) m->odd = 1;
+  if (!cols || threadIdx.x) return;
+  atomicMax(&m->i0, NPXa - lo);
+  atomicMax(&m->i1, hi + 1);
+  atomicMax(&m->j0, NPYa - (j + __builtin_ctzll(cols)));
+  atomicMax(&m->j1, j + 64 - __builtin_clzll(cols));
+}
+
+// The ring of cells that no step writes, zero in all nine arrays of a new second state (the
+// auxiliaries of its cells without UPML are formed before they are read).
+__global__ __launch_bounds__(256) void k_stream_ring(D2 *G, size_t stride, int NPXa, int NPYa)
+{
+  const int q = blockIdx.x * 256 + threadIdx.x, side = blockIdx.y, n = side < 2 ? NPYa : NPXa;
+  if (q >= n) return;
+  const size_t k = side < 2 ? (size_t)(side ? NPXa - 1 : 0) * NPYa + q : (size_t)q * NPYa + (side == 3 ? NPYa - 1 : 0);
+  for (int f = 0; f < 9; f++) ((D2 *)((char *)G + f * stride))[k] = d2(0, 0);
 }
 
 // ---------------------------------------------------------------- host
@@ -748,12 +771,12 @@ struct StreamState {
   fdtd_grid_desc d;
   int NPXa, NPYa, off;
   size_t ncell;
-  D2 *G;  // the nine arrays a launch writes, swapped with the grid's after it
+  D2 *G;  // the nine arrays a launch writes, swapped with the grid's after it; made by the first launch
   size_t stride;
-  double *ie[2];
+  double *ie[2];  // in one block
   double *xt, *yt;
   D2 *exy;
-  StreamMap *map;  // device, per 1/eps map
+  StreamMap *map;  // device, per 1/eps map; in one block with xt, yt and exy
   StreamMap seen;  // of all maps together
   StreamStrip *strips;  // interior, then frame
   int nint, nfrm;
@@ -782,20 +805,21 @@ int stream_create(const fdtd_grid_desc &d, int off, const Contour &ct, StreamSta
   s->NPYa = d.N_PY + 2 * off;
   s->ncell = (size_t)s->NPXa * s->NPYa;
   s->stride = stream_stride(s->ncell);
-  // a grid without room for a second state, or past 32-bit cell indexes, steps in place
+  // a grid without room for these, or past 32-bit cell indexes, steps in place
   if (s->ncell >= (size_t)1 << 31) return FDTD_ENOMEM;
-  bool room = dev_malloc(&s->G, 9 * s->stride) == hipSuccess;
-  for (int e = 0; e < (d.mode == FDTD_MODE_TM ? 1 : 2); e++)
-    room = room && dev_malloc(&s->ie[e], s->ncell * sizeof(double)) == hipSuccess;
-  room = room && dev_malloc(&s->xt, (size_t)s->NPXa * 8 * sizeof(double)) == hipSuccess &&
-         dev_malloc(&s->yt, (size_t)s->NPYa * 6 * sizeof(double)) == hipSuccess &&
-         dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)) == hipSuccess &&
-         dev_malloc(&s->map, 2 * sizeof(StreamMap)) == hipSuccess;
-  if (!room) {
+  const size_t X = s->NPXa, Y = s->NPYa, maps = d.mode == FDTD_MODE_TM ? 1 : 2;
+  char *b = nullptr;
+  const size_t tables = (X * 8 + Y * 6) * sizeof(double) + (X + Y) * sizeof(D2);
+  if (dev_malloc(&s->ie[0], maps * s->ncell * sizeof(double)) != hipSuccess ||
+      dev_malloc(&b, tables + 2 * sizeof(StreamMap)) != hipSuccess) {
     (void)hipGetLastError();
     return FDTD_ENOMEM;
   }
-  HIPCHK(hipMemsetAsync(s->G, 0, 9 * s->stride, 0));
+  if (maps > 1) s->ie[1] = s->ie[0] + s->ncell;
+  s->exy = (D2 *)b;
+  s->xt = (double *)(s->exy + X + Y);
+  s->yt = s->xt + X * 8;
+  s->map = (StreamMap *)(s->yt + Y * 6);
   s->ctot = ct.total;
   for (int q = 0; q < 4; q++) {
     const Seg &g = ct.s[q];
@@ -818,11 +842,7 @@ void stream_destroy(StreamState *s)
   if (!s) return;
   (void)dev_free(s->G);
   (void)dev_free(s->ie[0]);
-  (void)dev_free(s->ie[1]);
-  (void)dev_free(s->xt);
-  (void)dev_free(s->yt);
   (void)dev_free(s->exy);
-  (void)dev_free(s->map);
   (void)dev_free(s->strips);
   (void)dev_free(s->csamp);
   delete s;
@@ -834,7 +854,8 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   const int X = s->NPXa, Y = s->NPYa, off = s->off, T = STREAM_T;
   const bool tm = s->d.mode == FDTD_MODE_TM;
   const double c2 = 1.0 / s->d.mu0;
-  std::vector<double> xt((size_t)X * 8), yt((size_t)Y * 6);
+  std::vector<double> tab((size_t)X * 8 + (size_t)Y * 6);
+  double *const xt = tab.data(), *const yt = xt + (size_t)X * 8;
   std::vector<char> px(X, 0), py(Y, 0);
   for (int i = 0; i < X; i++) {
     const bool ring = i == 0 || i == X - 1;
@@ -883,25 +904,49 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   // the cells that keep auxiliaries: every updated one outside the box's rows or columns
   for (int i = 0; i < X; i++) xt[(size_t)i * 8 + 7] = i > 0 && i < X - 1 && (i < xlo || i >= xhi) ? 1.0 : 0.0;
   for (int j = 0; j < Y; j++) yt[5 * (size_t)Y + j] = j > 0 && j < Y - 1 && (j < ylo || j >= yhi) ? 1.0 : 0.0;
-  HIPCHK(hipMemcpy(s->xt, xt.data(), xt.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(s->yt, yt.data(), yt.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(s->xt, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
   // interior strips: every cell of their blocks lies in the box
   const int I0 = xlo + T, I1 = xhi - T, J0 = ylo + T, J1 = yhi - T;
   const bool inner = I0 < I1 && J0 < J1;
-  std::vector<StreamStrip> vi, vf;
-  auto band = [&](std::vector<StreamStrip> &v, int kind, int r0, int r1, int c0, int c1, int L) {
-    if (r0 >= r1 || c0 >= c1) return;
-    const int nch = std::max(1, (r1 - r0 + L - 1) / L), rows = (r1 - r0 + nch - 1) / nch;
-    for (int r = r0; r < r1; r += rows)
-      for (const Span &c : cover_cols(c0, c1, Y, kind ? 64 : 64 * stream_cols(s->d.mode, s->d.flavour), T, T)) {
+  struct Band {
+    int kind, r0, r1;
+    std::vector<Span> cols;
+  };
+  std::vector<Band> bands;
+  auto band = [&](int kind, int r0, int r1, int c0, int c1) {
+    if (r0 < r1 && c0 < c1)
+      bands.push_back({kind, r0, r1, cover_cols(c0, c1, Y, kind ? 64 : 64 * stream_cols(s->d.mode, s->d.flavour), T, T)});
+  };
+  if (inner) {  // the longer strips first
+    band(1, 1, I0, 1, Y - 1);
+    band(1, I1, X - 1, 1, Y - 1);
+    band(1, I0, I1, 1, J0);
+    band(1, I0, I1, J1, Y - 1);
+    band(0, I0, I1, J0, J1);
+  } else {
+    band(1, 1, X - 1, 1, Y - 1);
+  }
+  // rows of a band's strips of at most L, and how many of them
+  auto split = [](const Band &b, int L, int &nch) {
+    nch = std::max(1, (b.r1 - b.r0 + L - 1) / L);
+    const int rows = (b.r1 - b.r0 + nch - 1) / nch;
+    nch = (b.r1 - b.r0 + rows - 1) / rows;
+    return rows;
+  };
+  std::vector<StreamStrip> v;
+  auto fill = [&](const Band &b, int L) {
+    int nch;
+    const int rows = split(b, L, nch);
+    for (int r = b.r0; r < b.r1; r += rows)
+      for (const Span &c : b.cols) {
         StreamStrip t;
         memset(&t, 0, sizeof t);
-        t.kind = kind;
+        t.kind = b.kind;
         t.j0 = c.c0;
         t.j1 = c.c1;
         t.bj = c.b0;
         t.r0 = r;
-        t.r1 = std::min(r1, r + rows);
+        t.r1 = std::min(b.r1, r + rows);
         t.b0 = r == 1 ? 0 : r - T;
         t.bl = std::min(X - 1, t.r1 - 1 + T);
         t.s0 = t.r1;
@@ -926,32 +971,30 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
   // {24, 48} 71.1, apart 38.0 + 45.4 (since then 29.9 and 52.2 with the
   // chosen pairs).  Larger grids run the two kinds apart.
   static const int rows[][2] = {{8, 12}, {8, 16}, {16, 24}, {16, 32}, {24, 48}, {32, 64}, {64, 128}};
-  for (size_t q = 0; q < sizeof rows / sizeof rows[0]; q++) {
-    const int Lf = rows[q][0], Li = rows[q][1];
-    vi.clear();
-    vf.clear();
-    if (inner) {
-      band(vi, 0, I0, I1, J0, J1, Li);
-      band(vf, 1, 1, I0, 1, Y - 1, Lf);
-      band(vf, 1, I1, X - 1, 1, Y - 1, Lf);
-      band(vf, 1, I0, I1, 1, J0, Lf);
-      band(vf, 1, I0, I1, J1, Y - 1, Lf);
-    } else {
-      band(vf, 1, 1, X - 1, 1, Y - 1, Lf);
+  size_t q = 0;
+  for (; q + 1 < sizeof rows / sizeof rows[0]; q++) {
+    size_t all = 0;
+    for (const Band &b : bands) {
+      int nch;
+      split(b, rows[q][b.kind ? 0 : 1], nch);
+      all += nch * b.cols.size();
     }
-    if (vi.size() + vf.size() <= STREAM_BOTH_MAX) break;
+    if (all <= STREAM_BOTH_MAX) break;
   }
-  s->nint = (int)vi.size();
-  s->nfrm = (int)vf.size();
-  vf.insert(vf.end(), vi.begin(), vi.end());  // the longer strips first
+  for (const Band &b : bands) {
+    if (!b.kind) s->nfrm = (int)v.size();
+    fill(b, rows[q][b.kind ? 0 : 1]);
+  }
+  if (!inner) s->nfrm = (int)v.size();
+  s->nint = (int)v.size() - s->nfrm;
   (void)dev_free(s->strips);
   s->strips = nullptr;
   s->coefs = false;
-  if (dev_malloc(&s->strips, vf.size() * sizeof(StreamStrip)) != hipSuccess) {  // the grid steps in place
+  if (dev_malloc(&s->strips, v.size() * sizeof(StreamStrip)) != hipSuccess) {  // the grid steps in place
     (void)hipGetLastError();
     return FDTD_OK;
   }
-  HIPCHK(hipMemcpy(s->strips, vf.data(), vf.size() * sizeof(StreamStrip), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(s->strips, v.data(), v.size() * sizeof(StreamStrip), hipMemcpyHostToDevice));
   s->coefs = true;
   s->wave = false;
   return FDTD_OK;
@@ -959,16 +1002,15 @@ int stream_set_coefs(StreamState *s, const fdtd_coef_tables *t)
 
 int stream_set_eps(StreamState *s, double *const *eps)
 {
-  const dim3 blk(64, 4), grd((s->NPYa + 63) / 64, (s->NPXa + 3) / 4);
+  const dim3 blk(64, 4), grd((s->NPYa + 63) / 64, (s->NPXa + STREAM_IE_ROWS - 1) / STREAM_IE_ROWS);
   StreamMap m[2];
-  for (StreamMap &x : m) x = StreamMap{0, INT_MAX, -1, INT_MAX, -1};
-  HIPCHK(hipMemcpy(s->map, m, sizeof m, hipMemcpyHostToDevice));
+  HIPCHK(hipMemsetAsync(s->map, 0, sizeof m, 0));
   for (int e = 0; e < 2; e++)
     if (s->ie[e]) hipLaunchKernelGGL(k_stream_ie, grd, blk, 0, 0, eps[e], s->NPXa, s->NPYa, s->ie[e], s->map + e);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpy(m, s->map, sizeof m, hipMemcpyDeviceToHost));
-  s->seen = StreamMap{m[0].odd | m[1].odd, std::min(m[0].i0, m[1].i0), std::max(m[0].i1, m[1].i1),
-                      std::min(m[0].j0, m[1].j0), std::max(m[0].j1, m[1].j1)};
+  s->seen = StreamMap{m[0].odd | m[1].odd, std::max(m[0].i0, m[1].i0), std::max(m[0].i1, m[1].i1),
+                      std::max(m[0].j0, m[1].j0), std::max(m[0].j1, m[1].j1)};
   return FDTD_OK;
 }
 
@@ -1074,8 +1116,8 @@ int stream_few(const StreamState *s, int binned)
   double launch = (mpi ? 29 + 18e-6 * n : tm ? 40 + 16e-6 * n : 35 + 52e-6 * n) + (binned ? 13 : 0);
   const StreamMap &m = s->seen;
   const int h = 2 * STREAM_T;  // a frame strip reaches that far into the box
-  const bool frame = m.i0 < s->xlo + h || m.i1 >= s->xhi - h || m.j0 < s->ylo + h || m.j1 >= s->yhi - h;
-  if (m.i1 >= 0 && frame && n < 262144) launch += mpi ? 16 : tm ? 14 : 45;
+  const bool frame = s->NPXa - m.i0 < s->xlo + h || m.i1 > s->xhi - h || s->NPYa - m.j0 < s->ylo + h || m.j1 > s->yhi - h;
+  if (m.i1 && frame && n < 262144) launch += mpi ? 16 : tm ? 14 : 45;
   return std::min(STREAM_T, (int)(launch / step));
 }
 
@@ -1138,11 +1180,20 @@ static void launch(const StreamState *s, StreamArgs a)
 // buffer is swapped with the state's own); with at >= 0, the contour's samples
 // after every step in the entries [at, at + n) of the state's STREAM_SAMPLES, from
 // *smp on ([n][3][total]).  FDTD_ENOMEM, with nothing changed, if there is no room for these
+// or for the second state
 int stream_steps(StreamState *s, D2 **F, const fdtd_step_params *p, int n, int at, D2 **smp)
 {
   if (n < 1 || n > STREAM_T) return fdtd_fail(FDTD_EINVAL, "bad number of steps %d", n);
   const bool mpi = s->d.flavour == FDTD_FLAVOUR_MPI, tm = s->d.mode == FDTD_MODE_TM;
   const size_t entry = 3 * (size_t)s->ctot;
+  if (!s->G) {
+    if (dev_malloc(&s->G, 9 * s->stride) != hipSuccess) {
+      (void)hipGetLastError();
+      return FDTD_ENOMEM;
+    }
+    hipLaunchKernelGGL(k_stream_ring, dim3((std::max(s->NPXa, s->NPYa) + 255) / 256, 4), dim3(256), 0, 0, s->G, s->stride,
+                       s->NPXa, s->NPYa);
+  }
   if (at >= 0) {
     if (at + n > STREAM_SAMPLES) return fdtd_fail(FDTD_EINVAL, "bad sample entry %d", at);
     if (!s->csamp) {

@@ -319,9 +319,9 @@ struct SplitState {
   fdtd_grid_desc d;
   int ph, NPXa, NPYa;
   size_t ncell, stride;
-  D2 *G;  // the nine arrays a launch writes, swapped with the grid's after it
+  D2 *G;  // the nine arrays a launch writes, swapped with the grid's after it; made by the first launch
   double *cm, *xt, *yt;
-  D2 *exy;
+  D2 *exy;  // in one block with xt, yt
   SplitStrip *strips;
   int ns;
   bool coefs, cells, wave;
@@ -340,40 +340,41 @@ int split_create(const fdtd_grid_desc &d, SplitState **out)
   s->NPYa = d.N_PY;
   s->ncell = (size_t)s->NPXa * s->NPYa;
   s->stride = stream_stride(s->ncell);
-  // a grid without room for a second state, or past 32-bit cell indexes, steps in place
+  // a grid without room for these, or past 32-bit cell indexes, steps in place
   if (s->ncell >= (size_t)1 << 31) return FDTD_ENOMEM;
-  if (dev_malloc(&s->G, 9 * s->stride) != hipSuccess ||
-      dev_malloc(&s->cm, sp_ni(s->ph) * s->ncell * sizeof(double)) != hipSuccess ||
-      dev_malloc(&s->xt, (size_t)s->NPXa * 4 * sizeof(double)) != hipSuccess ||
-      dev_malloc(&s->yt, (size_t)s->NPYa * 3 * sizeof(double)) != hipSuccess ||
-      dev_malloc(&s->exy, (size_t)(s->NPXa + s->NPYa) * sizeof(D2)) != hipSuccess) {
+  const size_t nx = s->NPXa, ny = s->NPYa;
+  if (dev_malloc(&s->cm, sp_ni(s->ph) * s->ncell * sizeof(double)) != hipSuccess ||
+      dev_malloc(&s->exy, (nx + ny) * sizeof(D2) + (nx * 4 + ny * 3) * sizeof(double)) != hipSuccess) {
     (void)hipGetLastError();
     return FDTD_ENOMEM;
   }
-  HIPCHK(hipMemsetAsync(s->G, 0, 9 * s->stride, 0));
+  s->xt = (double *)(s->exy + nx + ny);
+  s->yt = s->xt + nx * 4;
   // Strips: a halo of T cells below and left, T + 1 above and right (the non-standard TE
   // half reaches one cell further there).  Rows per strip as in fdtd_stream.hip: the
   // shortest strips that all run at once, two workgroups on each of 256 compute units.
   const int T = sp_t(s->ph), X = s->NPXa, Y = s->NPYa;
-  std::vector<SplitStrip> v;
+  const std::vector<Span> cols = cover_cols(1, Y - 1, Y, 64, T, T + 1);
+  int rows = 0;
   for (int L : {8, 12, 16, 24, 32, 48, 64, 96, 128}) {
-    v.clear();
-    const int nch = (X - 2 + L - 1) / L, rows = (X - 2 + nch - 1) / nch;
-    for (int r = 1; r < X - 1; r += rows)
-      for (const Span &c : cover_cols(1, Y - 1, Y, 64, T, T + 1)) {
-        SplitStrip q;
-        q.j0 = c.c0;
-        q.j1 = c.c1;
-        q.bj = c.b0;
-        q.r0 = r;
-        q.r1 = std::min(X - 1, r + rows);
-        q.b0 = r == 1 ? 0 : r - T;
-        q.bl = std::min(X - 1, q.r1 + T);
-        q.pad = 0;
-        v.push_back(q);
-      }
-    if (v.size() <= 512) break;
+    const int nch = (X - 2 + L - 1) / L;
+    rows = (X - 2 + nch - 1) / nch;
+    if ((X - 2 + rows - 1) / rows * cols.size() <= 512) break;
   }
+  std::vector<SplitStrip> v;
+  for (int r = 1; r < X - 1; r += rows)
+    for (const Span &c : cols) {
+      SplitStrip q;
+      q.j0 = c.c0;
+      q.j1 = c.c1;
+      q.bj = c.b0;
+      q.r0 = r;
+      q.r1 = std::min(X - 1, r + rows);
+      q.b0 = r == 1 ? 0 : r - T;
+      q.bl = std::min(X - 1, q.r1 + T);
+      q.pad = 0;
+      v.push_back(q);
+    }
   s->ns = (int)v.size();
   if (dev_malloc(&s->strips, v.size() * sizeof(SplitStrip)) != hipSuccess) {
     (void)hipGetLastError();
@@ -388,8 +389,6 @@ void split_destroy(SplitState *s)
   if (!s) return;
   (void)dev_free(s->G);
   (void)dev_free(s->cm);
-  (void)dev_free(s->xt);
-  (void)dev_free(s->yt);
   (void)dev_free(s->exy);
   (void)dev_free(s->strips);
   delete s;
@@ -398,7 +397,8 @@ void split_destroy(SplitState *s)
 int split_set_coefs(SplitState *s, const fdtd_coef_tables *t)
 {
   const int X = s->NPXa, Y = s->NPYa;
-  std::vector<double> xt((size_t)X * 4, 0.0), yt((size_t)Y * 3, 0.0);
+  std::vector<double> tab((size_t)X * 4 + (size_t)Y * 3, 0.0);
+  double *const xt = tab.data(), *const yt = xt + (size_t)X * 4;
   const double mu = s->d.mu0;
   auto coef = [&](double sig) { return (1.0 - sig / mu) / (1.0 + sig / mu); };
   const bool ns = s->ph == NS_TM || s->ph == NS_TE;
@@ -415,8 +415,7 @@ int split_set_coefs(SplitState *s, const fdtd_coef_tables *t)
     yt[(size_t)Y + j] = ns ? t->y[1][j] : coef(t->y[1][j]);
     yt[2 * (size_t)Y + j] = ns || ring ? 0.0 : 1.0 / (mu + t->y[1][j]);
   }
-  HIPCHK(hipMemcpy(s->xt, xt.data(), xt.size() * sizeof(double), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(s->yt, yt.data(), yt.size() * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(s->xt, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
   s->coefs = true;
   return FDTD_OK;
 }
@@ -459,9 +458,18 @@ int split_few(const SplitState *s)
   return n < (size_t)1 << 16 && s->ph == NS_TM ? 3 : n < (size_t)1 << 18 ? 2 : n < (size_t)8 << 20 ? 1 : 0;
 }
 
-// n <= split_depth() steps of one wave direction from *F, which then holds the new state
+// n <= split_depth() steps of one wave direction from *F, which then holds the new state;
+// FDTD_ENOMEM, with nothing changed, if there is no room for the second state
 int split_steps(SplitState *s, D2 **F, const fdtd_step_params *p, int n)
 {
+  if (!s->G) {
+    if (dev_malloc(&s->G, 9 * s->stride) != hipSuccess) {
+      (void)hipGetLastError();
+      return FDTD_ENOMEM;
+    }
+    // (the ring and the arrays these solvers do not use stay zero)
+    HIPCHK(hipMemsetAsync(s->G, 0, 9 * s->stride, 0));
+  }
   const double rad = p->angle_deg * M_PI / 180.0, kx = cos(rad) * p->k, ky = sin(rad) * p->k;
   if (!s->wave || p->angle_deg != s->angle || p->k != s->k) {
     std::vector<D2> t(s->NPXa + s->NPYa);
