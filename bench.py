@@ -482,8 +482,8 @@ def run_solvers_fp64(args, m):
     """Every solver of enum SOLVER in FP64 on the mie1056
     grid (the reference's cylinder; CW source for the MPI, split-field and NS
     solvers, Gaussian pulse for the plain UPML ones), without the per-step NTFF:
-    the step rate of each over `steps` simulator_calc() calls after 20 untimed
-    ones.  Not the headline: a measurement of the solvers beside the UPML path,
+    the step rate of each over one fdtd_simulator_run of `steps` steps after 20
+    untimed ones.  Not the headline: a measurement of the solvers beside the UPML path,
     whose kernel durations a rocprofv3 kernel trace of this command gives."""
     import numpy as np
     L = m.lib()

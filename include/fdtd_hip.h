@@ -160,8 +160,13 @@ int fdtd_hip_grid_set_ns_coefs(fdtd_grid *g, const double *cells, double r_half)
 int fdtd_hip_grid_form_ns_coefs(fdtd_grid *g, const double *const sig[4], double omega, double k, double r_half);
 /* one reference update(): E/H halves, source, per-step NTFF */
 int fdtd_hip_grid_step(fdtd_grid *g, const fdtd_step_params *p);
-/* n update()s, p[i] the parameters of the i-th: the same results as n calls of
- * fdtd_hip_grid_step; FP64 grids advance several steps per launch */
+/* n update()s, p[i] the parameters of the i-th.  FP64 grids advance several steps
+ * per launch where n is large enough for that to cost less; a call of few steps,
+ * and a grid the blocked steps cannot take (a restored state, a cell of infinite
+ * or very large permittivity, no memory for their second state), goes by the
+ * kernels of one step.  The two round differently (contraction, order of the
+ * terms), so FP64 results agree with n calls of fdtd_hip_grid_step to rounding,
+ * not bit by bit. */
 int fdtd_hip_grid_steps(fdtd_grid *g, const fdtd_step_params *p, int n);
 /* which 0..8: TM Ez Jz Dz Hx Mx Bx Hy My By / TE Ex Jx Dx Ey Jy Dy Hz Mz Bz;
  * host buffers hold NPXa*NPYa complex doubles (re,im) in the solver layout */

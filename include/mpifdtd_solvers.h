@@ -202,8 +202,9 @@ void fdtd_solver_setNTFFTime(int on);
 void fdtd_solver_setFileOutput(int on);
 /* dims of the active solver: NPXa, NPYa, off, arraySize */
 int fdtd_solver_dims(int out[4]);
-/* FDTD_FP64 (default): FP64 kernels, several steps per launch; FDTD_FP32: fused FP32
- * kernels with temporal blocking (set before init).  Getters return double
+/* FDTD_FP64 (default): FP64 kernels, several steps per launch where a call runs enough
+ * of them (a run cut into other calls agrees to rounding, not bit by bit); FDTD_FP32:
+ * fused FP32 kernels with temporal blocking (set before init).  Getters return double
  * complex in both cases. */
 void fdtd_solver_setPrecision(int precision);
 int fdtd_solver_getPrecision(void);

@@ -65,7 +65,7 @@ struct StreamArgs {
   const double *yt;         // [6][NPYa] column coefficients
   const D2 *ex, *ey;        // e^{i kx x}, e^{i ky y} (plain: of the pulse's carrier)
   const StreamStrip *strips;
-  int ns, NPXa, NPYa, off, T;
+  int ns, NPXa, NPYa, T;
   int xlo, xhi;             // rows without UPML
   double c2, mu0;
   // sources: entry 0 the step before the launch's first, then its steps
@@ -636,13 +636,13 @@ __device__ __forceinline__ void strip_body(const StreamArgs &a, const StreamStri
         const int O = (u - S + 2 * NS) % NS;
         if (last) store(O, n - S);
         else put(O, it & 1);
-        if (K > 1) lds_barrier();
+        lds_barrier();
       }
     }
   };
-  if (w == 0) march(std::true_type(), std::integral_constant<bool, K == 1>());
+  if (w == 0) march(std::true_type(), std::false_type());
   else if (w == K - 1) march(std::false_type(), std::true_type());
-  else if (K > 2) march(std::false_type(), std::false_type());
+  else march(std::false_type(), std::false_type());
 }
 
 template <int MODE, int FLAV, int PML, int C, int S, int PF>
@@ -1136,7 +1136,6 @@ static void fill_args(const StreamState *s, StreamArgs &a, const D2 *src, D2 *ds
   a.ey = s->exy + s->NPXa;
   a.NPXa = s->NPXa;
   a.NPYa = s->NPYa;
-  a.off = s->off;
   a.xlo = s->xlo;
   a.xhi = s->xhi;
   a.c2 = 1.0 / d.mu0;
