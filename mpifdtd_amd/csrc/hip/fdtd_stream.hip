@@ -19,10 +19,10 @@
 // for (stream_fill_aux).  Strips of the frame run the full recurrences; in their
 // cells without UPML the auxiliaries are formed from the fields as a row is
 // loaded.  What bounds it: the chain of a row's dependent FP64 operations, LDS
-// hand-ons and one barrier per row (the two kernels keep their SIMDs about 45 %
-// active, waves waiting 40-50 % of the time), at 7.3 us a step on 1056 x 1056 where the
-// two-launch step that reads and writes every array took 57 (8-step launches of
-// 58.5 us, TM; two columns a lane: one took 38.0 + 45.4 us in two launches).
+// hand-ons and one barrier per row (counters of MPI TM on 1056 x 1056: a busy compute
+// unit's VALU works 47 % of the time, its waves wait 39 % of theirs, HBM traffic
+// 3.3 TB/s), at 6.7 us a step on 1056 x 1056 where the two-launch step that reads and
+// writes every array took 57 (8-step launches of 53 us, TM).
 // Physics per step as in the reference (mpiTM_UPML.c:196-217,
 // mpiTE_UPML.c:290-304, fdtdTM_upml.c:54-66, fdtdTE_upml.c:168-192).
 #include <hip/hip_runtime.h>
